@@ -137,6 +137,8 @@ SIGNATURES = {
     "gx_bins_clear": [_P, _P, _I, _P],
     "gx_bins_finalize": [_P, _P, _I, _D, _I, _I, _D, _D, _D, POINTER(c_double), _D, _P, _P, _P],
     "gx_detector_accumulate": [POINTER(GxDetector), _P],
+    "gx_detector_work_size": [POINTER(GxDetector), POINTER(c_int64)],
+    "gx_detector_accumulate_ws": [POINTER(GxDetector), _P, _P],
     "gx_detector_finalize": [_P, _I, _I, _I, _P, _P],
     "gx_rotate_points": [POINTER(c_double), _P, _P, _P, _I, _P, _P, _P, _P],
     "gx_intersect": [_P, _I, _I, _I, _D, _D, _D, _D, _P, _P, _P, _I, _D, _I, _P, _P],

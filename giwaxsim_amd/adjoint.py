@@ -40,7 +40,7 @@ import torch
 from . import _lib
 from ._lib import GxAdjoint, GxDetector, GxFrames, GxSlab, call
 from .engine import (_empty, bin_scale_for, chirpz_adjoint_tables, chirpz_band_tables, chirpz_bands,
-                     chirpz_tables, collapse_records, detector_plan, device, element_table,
+                     chirpz_tables, collapse_records, detector_plan, detector_work, device, element_table,
                      fft_precision, frame_plan, gauss_prefix, intensity_bound, is_pow2_grid,
                      pixels_per_bin, ptr, stream_handle, twiddles)
 from .tools.ptable_dict import aff_dict, ptable
@@ -224,6 +224,7 @@ class DifferentiableSlab:
             orient_w=ptr(self.det_ow).value, iq=ptr(self.iq64).value, iq_f64=1,
             cy=g.c_n, cx=g.c_n, cz=g.c_n, qx_min=float(np.min(ax)), qy_min=float(np.min(ax)),
             qz_min=float(np.min(ax)), dq=float(np.diff(ax)[0]), det=ptr(self.det_raw).value)
+        self.det_lin = detector_work(self.detector_desc)
         # the detector adjoint goes through a transpose map of the orientation gather
         # when it fits (<= 32 GB of runs of pixels, 9 bytes a run, of the 288 GB of HBM),
         # else scatters into copies of its accumulator (<= 256 MB)
@@ -441,7 +442,7 @@ class DifferentiableSlab:
         aff = _lib.dbl_array(aff_dict['C'])
         call("gx_bins_finalize", ptr(self.bin_sum), ptr(self.bin_cnt), g.c_n, self.bin_scale, g.c_lo,
              g.q_num, start, step, stop, aff, float(ptable['C']), ptr(self.iq64), ptr(None), st)
-        call("gx_detector_accumulate", ctypes.byref(self.detector_desc), st)
+        call("gx_detector_accumulate_ws", ctypes.byref(self.detector_desc), ptr(self.det_lin), st)
         call("gx_detector_finalize", ptr(self.det_raw), self.n_pix, self.n_pix, self._flags(),
              ptr(self.det_out), st)
 

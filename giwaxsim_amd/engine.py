@@ -1054,6 +1054,13 @@ def detector_plan(num_pixels, max_q, angle_init_vals, angle_init_axs, psis, psi_
                         orient_w=np.array(ws, dtype=np.float64))
 
 
+def detector_work(desc):
+    """The work buffer of gx_detector_accumulate_ws for a detector descriptor."""
+    n = ctypes.c_int64(0)
+    call("gx_detector_work_size", ctypes.byref(desc), ctypes.byref(n))
+    return _empty(n.value, torch.float64)
+
+
 def run_detector(iq_dev, qx, qy, qz, plan: DetectorPlan, mirror, floor_scale=True):
     """Orientation sum + finalize on the device.  ``iq_dev``: float32 or float64
     device tensor [cy, cx, cz].  Returns the FP64 device image [n, n] (mirrored when
@@ -1077,7 +1084,8 @@ def run_detector(iq_dev, qx, qy, qz, plan: DetectorPlan, mirror, floor_scale=Tru
                    qx_min=float(np.min(qx)), qy_min=float(np.min(qy)), qz_min=float(np.min(qz)),
                    dq=float(dq), det=ptr(det).value)
     st = stream_handle()
-    call("gx_detector_accumulate", ctypes.byref(d), st)
+    work = detector_work(d)
+    call("gx_detector_accumulate_ws", ctypes.byref(d), ptr(work), st)
     out = _empty(n * n, torch.float64)
     flags = (_lib.GX_FIN_FLOOR_SCALE if floor_scale else 0) | (_lib.GX_FIN_MIRROR if mirror else 0)
     call("gx_detector_finalize", ptr(det), n, n, flags, ptr(out), st)

@@ -284,6 +284,12 @@ int gx_bins_finalize(const unsigned long long *bin_sum, const int32_t *bin_cnt, 
  * orientations, tools/detector.py:234-244, 278-300; intersect_detector
  * 194-232), accumulated in FP64 in (psi, phi, theta) order. */
 int gx_detector_accumulate(const gx_detector *d, gx_stream_t stream);
+/* gx_detector_accumulate, bit for bit and faster, with a 64-byte aligned work buffer for
+ * per-orientation linear index maps, which replace the rotations of every sample.
+ * gx_detector_work_size gives its size in doubles from the descriptor (host only; 0 where
+ * the maps do not apply and the plain kernels run). */
+int gx_detector_work_size(const gx_detector *d, int64_t *n_doubles);
+int gx_detector_accumulate_ws(const gx_detector *d, double *work, gx_stream_t stream);
 /* flags & GX_FIN_MIRROR: mirror_vertical_horizontal (tools/detector.py:246-275);
  * then flags & GX_FIN_FLOOR_SCALE: NaN -> 1e-6, <= 0 -> 1e-6, * 1e-6
  * (tools/comparison.py:857-868).  det and out must not alias. */
