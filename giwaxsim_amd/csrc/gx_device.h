@@ -181,6 +181,86 @@ template <typename C> struct Dft<16, C> {
   }
 };
 
+// Dft<R> whose inputs v[NZ ..] are zero (they are not read): the same operations without
+// those on zeros, in the same order.
+template <int R, int NZ, typename C> struct DftHead;
+template <int NZ, typename C> struct DftHead<4, NZ, C> {
+  static __device__ __forceinline__ void run(C *v) {
+    const C z = C{0, 0};
+    if constexpr (NZ >= 4) {
+      Dft<4, C>::run(v);
+    } else if constexpr (NZ <= 0) {
+      v[0] = v[1] = v[2] = v[3] = z;
+    } else if constexpr (NZ == 1) {
+      v[1] = v[2] = v[3] = v[0];
+    } else {
+      const C t0 = NZ > 2 ? cadd(v[0], v[2]) : v[0], t1 = NZ > 2 ? csub(v[0], v[2]) : v[0];
+      const C t2 = v[1], t3 = cmul_mi(v[1]);
+      v[0] = cadd(t0, t2);
+      v[2] = csub(t0, t2);
+      v[1] = cadd(t1, t3);
+      v[3] = csub(t1, t3);
+    }
+  }
+};
+template <int NZ, typename C> struct DftHead<8, NZ, C> {
+  static __device__ __forceinline__ void run(C *v) {
+    if constexpr (NZ >= 8) {
+      Dft<8, C>::run(v);
+    } else {
+      using T = typename Real<C>::T;
+      const T c = (T)0.70710678118654752440;
+      C e[4] = {v[0], v[2], v[4], v[6]};
+      C o[4] = {v[1], v[3], v[5], v[7]};
+      DftHead<4, (NZ + 1) / 2, C>::run(e);
+      DftHead<4, NZ / 2, C>::run(o);
+      if constexpr (NZ / 2 > 0) {
+        C w1 = C{c * (o[1].x + o[1].y), c * (o[1].y - o[1].x)};
+        C w2 = cmul_mi(o[2]);
+        C w3 = C{c * (o[3].y - o[3].x), -c * (o[3].x + o[3].y)};
+        v[0] = cadd(e[0], o[0]);
+        v[4] = csub(e[0], o[0]);
+        v[1] = cadd(e[1], w1);
+        v[5] = csub(e[1], w1);
+        v[2] = cadd(e[2], w2);
+        v[6] = csub(e[2], w2);
+        v[3] = cadd(e[3], w3);
+        v[7] = csub(e[3], w3);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = v[i + 4] = e[i];
+      }
+    }
+  }
+};
+template <int NZ, typename C> struct DftHead<16, NZ, C> {
+  static __device__ __forceinline__ void run(C *v) {
+    if constexpr (NZ >= 16) {
+      Dft<16, C>::run(v);
+    } else {
+      using T = typename Real<C>::T;
+      const T c1 = (T)0.92387953251128675613, s1 = (T)0.38268343236508977173;
+      const T c2 = (T)0.70710678118654752440;
+      C e[8], o[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        e[i] = v[2 * i];
+        o[i] = v[2 * i + 1];
+      }
+      DftHead<8, (NZ + 1) / 2, C>::run(e);
+      DftHead<8, NZ / 2, C>::run(o);
+      const C w[8] = {C{(T)1, (T)0}, C{c1, -s1}, C{c2, -c2}, C{s1, -c1},
+                      C{(T)0, (T)-1}, C{-s1, -c1}, C{-c2, -c2}, C{-c1, -s1}};
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        C t = (k == 0) ? o[0] : (k == 4 ? cmul_mi(o[4]) : cmul(o[k], w[k]));
+        v[k] = cadd(e[k], t);
+        v[k + 8] = csub(e[k], t);
+      }
+    }
+  }
+};
+
 // ------------------------------------------------------------------------------------
 // In-wave Stockham autosort FFT.  One transform of N points per wave; each of
 // the 64 lanes holds P = N/64 points in registers.  A stage of radix R with
@@ -520,6 +600,76 @@ __device__ __forceinline__ void chirpz_block(C (&v)[M / GX_BLK_FFT], C *lds, con
   fft_block<M, C>(v, lds, tw, tid);
 #pragma unroll
   for (int q = 0; q < P; ++q) v[q] = C{v[q].x, -v[q].y};
+}
+
+// ------------------------------------------------------------------------------------
+// The zoomed chirp-z band transform of length 1024 within one wave (16 points per lane,
+// radices 16.4.16: the first and last agree, so lane l holds points l + 64 r before and
+// after a transform).  No block barriers and three stages per transform, against five stages
+// of four points per thread and twenty barriers a row of a block-wide transform of this length.
+// ------------------------------------------------------------------------------------
+constexpr int CHW_M = 1024, CHW_P = CHW_M / GX_WAVE;
+constexpr int CHW_BUF = CHW_M + CHW_M / 16;  // complex values of a wave's exchange buffer
+// The first butterflies have a form for inputs of up to CHW_NZ groups of 64 points, and the
+// kernels are compiled for bands of up to CHW_G groups and for all 16: at the fit geometry 603
+// rows and 290 frequencies (10 and 5 groups).
+constexpr int CHW_NZ = 10, CHW_G = 5;
+
+// The transform after its first butterflies (DftHead<16> on v[r] = x[lane + 64 r], which the
+// caller runs for as many inputs as may not be zero) -> v[r] = X[lane + 64 r]; the buffer is
+// free again on return.  Both exchanges keep immediate offsets and conflict-free banks:
+// element i of the first sits at i + i / 16, of the second at i with bit 4 flipped in odd
+// groups of 64.
+template <typename C>
+__device__ __forceinline__ void fft_wave_1024_tail(C (&v)[CHW_P], C *lds, const C *__restrict__ tw, int lane) {
+#pragma unroll
+  for (int r = 0; r < 16; ++r) lds[lane * 17 + r] = v[r];
+  wave_sync();
+  {
+    const C *p = lds + lane + lane / 16;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[4 * t + r] = p[68 * t + 272 * r];
+  }
+  wave_sync();
+  fft_butterflies<CHW_M, 4, 16, CHW_P, C>(v, tw, lane);
+  {
+    // butterfly j = lane + 64 t stores element (j / 16) 64 + j % 16 + 16 r; j / 16 = lane / 16 + 4 t
+    const int g = lane / 16;
+    C *p = lds + g * 64 + (lane & 15);
+    C *even = (g & 1) ? p + 16 : p, *odd = (g & 1) ? p : p + 16;  // r = 0 (2) and r = 1 (3)
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) ((r & 1) ? odd : even)[256 * t + 32 * (r / 2)] = v[4 * t + r];
+  }
+  wave_sync();
+  {
+    const C *even = lds + lane, *odd = lds + (lane ^ 16);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = ((r & 1) ? odd : even)[64 * r];
+  }
+  wave_sync();
+  fft_butterflies<CHW_M, 16, 64, CHW_P, C>(v, tw, lane);
+}
+
+// The circular convolution of chirpz_block on a wave, the input after its first butterflies
+// (DftHead<16>); a caller that uses only the first outputs v[0 .. G - 1] pays for those of the
+// last stage only.
+template <typename C>
+__device__ __forceinline__ void chirpz_wave(C (&v)[CHW_P], C *lds, const C *__restrict__ K, const C *__restrict__ tw,
+                                            int lane) {
+  fft_wave_1024_tail<C>(v, lds, tw, lane);
+#pragma unroll
+  for (int r = 0; r < CHW_P; ++r) {
+    const C x = cmul(v[r], K[lane + GX_WAVE * r]);
+    v[r] = C{x.x, -x.y};
+  }
+  DftHead<16, 16, C>::run(v);
+  fft_wave_1024_tail<C>(v, lds, tw, lane);
+#pragma unroll
+  for (int r = 0; r < CHW_P; ++r) v[r] = C{v[r].x, -v[r].y};
 }
 
 // ------------------------------------------------------------------------------------

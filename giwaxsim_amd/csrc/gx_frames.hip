@@ -1543,6 +1543,239 @@ void k_rowpass_bs(gx_frames d, int64_t f0) {
   }
 }
 
+// The row pass for bands of length 1024: a wave per row (chirpz_wave), the block's four rows
+// stored transposed.  G: 64-value groups of the band (bs_rk <= 64 G).
+//
+// The block-wide form spent a row in 20 block barriers at four points per thread.  Here a row
+// stays in one wave's registers and private LDS, its four rows share the masked chirp in LDS
+// (FP32), and the band is staged in the exchange buffers, so four blocks share a CU: 556,000
+// rows at N = 1048 (fit geometry, FP32) 4.22 -> 1.89 ms, about 1,700 vector instructions a row
+// at 90% of their issue rate.  More rows per wave one after another were slower (their table
+// indices held 50 more registers: two rows 4.5 ms per evaluation against 3.2).
+template <typename C, int G>
+__global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(sizeof(C) == 8 ? 4 : 2)))
+void k_rowpass_bsw(gx_frames d, int64_t f0) {
+  GX_RESOLVE_AVG(d);
+  using T = typename Real<C>::T;
+  constexpr int RB = BLK / GX_WAVE;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int lane = threadIdx.x & (GX_WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / GX_WAVE);
+  C *bufs = reinterpret_cast<C *>(smem_raw), *fbuf = bufs + wave * CHW_BUF;
+  C *cm = bufs + RB * CHW_BUF;  // [1024] chirp times the smoothed y mask
+  int32_t *acc_re = reinterpret_cast<int32_t *>(fbuf), *acc_im = acc_re + CHW_M;
+  const int N = (int)d.N;
+  const int fb = blockIdx.y;
+  const double *fp = d.fparams + (f0 + fb) * GX_FP_STRIDE;
+  const int jlo = (int)fp[GX_FP_JLO], jhi = (int)fp[GX_FP_JHI];
+  const int wf = jhi - jlo + 1;
+  if (wf <= 0) return;  // block-uniform
+  const int32_t *bnd = d.idx_bounds + 4 * fb;
+  if (wf > d.W || jlo < d.bs_rlo + N / 2 || jhi > d.bs_rlo + d.bs_rk - 1 + N / 2 ||
+      (bnd[1] != INT_MIN && bnd[1] > d.bs_M - d.bs_rk)) {  // as k_rowpass_bs
+    if (threadIdx.x == 0 && blockIdx.x == 0) atomicAdd(&d.status[1], 1);
+    return;
+  }
+  const C *chirp = reinterpret_cast<const C *>(d.bs_chirp);
+  const int z0 = blockIdx.x * RB, z = z0 + wave;
+  const int zlo = bnd[2], zhi = bnd[3];
+  const bool inside = !d.fill_bkg || (z >= zlo && z < zhi);
+  const int a0 = d.row_off[z], a1 = d.row_off[z + 1];  // Z is a multiple of 8
+  const bool atoms = inside && a1 > a0;                // wave-uniform
+  if (atoms) {
+#pragma unroll
+    for (int i = 0; i < (2 * CHW_M) / (4 * GX_WAVE); ++i)
+      reinterpret_cast<int4 *>(acc_re)[lane + GX_WAVE * i] = make_int4(0, 0, 0, 0);
+  }
+  const bool head = bnd[1] < GX_WAVE * CHW_NZ;  // the frame's atoms end below (block-uniform)
+  auto chirp_mask = [&](int n) {
+    C x = C{(T)0, (T)0};
+    if (n < N) {
+      x = chirp[n];
+      if (d.smooth) {
+        const T m = (T)d.col_sy[(int64_t)fb * N + n];
+        x = C{x.x * m, x.y * m};
+      }
+    }
+    return x;
+  };
+  // shared by the block's rows in FP32; in FP64 the table would leave one block per CU
+  if constexpr (sizeof(C) == 8) {
+#pragma unroll
+    for (int i = 0; i < CHW_M / BLK; ++i) {
+      const int n = threadIdx.x + BLK * i;
+      if (!(head && n >= GX_WAVE * CHW_NZ)) cm[n] = chirp_mask(n);
+    }
+    __syncthreads();
+  } else {
+    wave_sync();
+  }
+  C v[CHW_P];
+  if (atoms) {
+    const double s = fp[GX_FP_SIN], c = fp[GX_FP_COS];
+    const double ymin = dkey_inv(d.ymin_key[3 * fb]);
+    // every deposited y is at most y_max <= bs_M - bs_rk < 1024 (checked above)
+    const int ylo = bnd[0], yhi = bnd[1];
+    const int ya = d.fill_bkg ? (ylo == INT_MAX ? N : ylo + 1) : 0;
+    const int yb = min(d.fill_bkg ? (yhi == INT_MIN ? 0 : yhi) : N, CHW_M);
+    const double r = d.r, rinv = 1.0 / d.r;
+    for (int a = a0 + lane; a < a1; a += GX_WAVE * SCATTER_UNROLL) {
+      double xs[SCATTER_UNROLL], ys[SCATTER_UNROLL];
+      int2 qs[SCATTER_UNROLL];
+#pragma unroll
+      for (int u = 0; u < SCATTER_UNROLL; ++u) {
+        const int au = a + u * GX_WAVE;
+        const bool ok = au < a1;
+        xs[u] = ok ? d.ax[au] : 0.0;
+        ys[u] = ok ? d.ay[au] : 0.0;
+        qs[u] = ok ? reinterpret_cast<const int2 *>(d.aq)[au] : make_int2(0, 0);
+      }
+#pragma unroll
+      for (int u = 0; u < SCATTER_UNROLL; ++u) {
+        if (a + u * GX_WAVE >= a1) break;
+        const double yy = (xs[u] * s + ys[u] * c) - ymin;
+        const int yi = floor_div_in(yy, r, rinv, ya, yb);
+        if (yi >= 0) {
+          atomicAdd(&acc_re[yi], qs[u].x);
+          atomicAdd(&acc_im[yi], qs[u].y);
+        }
+      }
+    }
+    wave_sync();
+    const T inv = (T)ldexp(1.0, -d.row_exp[z]);
+    auto load = [&](int q) {
+      const int n = lane + GX_WAVE * q;
+      v[q] = cmul(C{(T)acc_re[n] * inv, (T)acc_im[n] * inv}, sizeof(C) == 8 ? cm[n] : chirp_mask(n));
+    };
+    if (head) {
+#pragma unroll
+      for (int q = 0; q < CHW_NZ; ++q) load(q);
+      DftHead<16, CHW_NZ, C>::run(v);
+    } else {
+#pragma unroll
+      for (int q = 0; q < CHW_P; ++q) load(q);
+      DftHead<16, CHW_P, C>::run(v);
+    }
+    wave_sync();
+    chirpz_wave<C>(v, fbuf, reinterpret_cast<const C *>(d.bs_kernel),
+                       reinterpret_cast<const C *>(d.bs_twiddle), lane);
+    wave_sync();
+  }
+  // the band, staged in the wave's buffer
+  const bool dense = d.fill_bkg || d.smooth;
+  const double avv_re = d.avg_re * d.max_voxels, avv_im = d.avg_im * d.max_voxels;
+  const double mz = d.smooth ? d.col_sz[(int64_t)fb * N + z] : 1.0;
+  const C *spec = reinterpret_cast<const C *>(d.col_spec) + (int64_t)fb * d.W;
+#pragma unroll
+  for (int q = 0; q < G; ++q) {
+    const int j = lane + GX_WAVE * q;
+    if (j >= (int)d.bs_rk) continue;
+    const int k = (int)d.bs_rlo + j;   // signed frequency, -N/2 <= k < N - N/2
+    const int w = k + N / 2 - jlo;     // fftshifted column within the frame's band
+    if (w < 0 || w >= wf) continue;
+    C o = C{(T)0, (T)0};
+    if (atoms) o = cmul(v[q], chirp[k < 0 ? -k : k]);
+    if (!inside) {
+      o = (k == 0) ? C{(T)(avv_re * (double)N), (T)(avv_im * (double)N)} : C{(T)0, (T)0};
+    } else if (dense) {
+      const C u = spec[w];
+      double ore = mz * ((double)o.x + (double)u.x);
+      double oim = mz * ((double)o.y + (double)u.y);
+      if (d.smooth && k == 0) {
+        ore = ore + avv_re * (double)N;
+        oim = oim + avv_im * (double)N;
+      }
+      o = C{(T)ore, (T)oim};
+    }
+    fbuf[w] = o;
+  }
+  __syncthreads();
+  C *out = reinterpret_cast<C *>(d.inter) + (int64_t)fb * d.W * d.Z + z0;
+  for (int idx = threadIdx.x; idx < wf * RB; idx += BLK) {
+    const int w = idx / RB, q = idx - w * RB;
+    out[(int64_t)w * d.Z + q] = bufs[q * CHW_BUF + w];
+  }
+}
+
+// The column pass for bands of length 1024: a wave per kept column, no block barriers (fit
+// geometry, 200,000 columns: 1.10 -> 0.81 ms; the atomics take 0.2 ms of it).  The k = 0
+// column's background A N is subtracted on every row and its transform, A N^2 at k_z = 0, added:
+// it needs no tail beyond the band and does not cancel in FP32 (its weak voxels' error 2e-5 ->
+// under 1e-5 of themselves).
+template <typename C, int G>
+__global__ __launch_bounds__(BLK) void k_colpass_bsw(gx_frames d, int64_t f0) {
+  GX_RESOLVE_AVG(d);
+  using T = typename Real<C>::T;
+  __shared__ C lds[BLK / GX_WAVE][CHW_BUF];
+  const int N = (int)d.N;
+  const int lane = threadIdx.x & (GX_WAVE - 1);
+  const int wave = threadIdx.x / GX_WAVE;
+  const int fb = blockIdx.y;
+  const double *fp = d.fparams + (f0 + fb) * GX_FP_STRIDE;
+  const int jlo = (int)fp[GX_FP_JLO], jhi = (int)fp[GX_FP_JHI];
+  const int wcol = blockIdx.x * (BLK / GX_WAVE) + wave;
+  if (wcol > jhi - jlo || wcol >= d.W) return;  // wave-uniform; no block barrier below
+  const int j = jlo + wcol;
+  const double hx = (j == N - 1) ? fp[GX_FP_HX_STOP] : (double)j * fp[GX_FP_HX_STEP] + fp[GX_FP_HX_START];
+  const double hy = (j == N - 1) ? fp[GX_FP_HY_STOP] : (double)j * fp[GX_FP_HY_STEP] + fp[GX_FP_HY_START];
+  const double dqinv = 1.0 / d.dq;
+  const long long bx = to_int(floor_div(hx - d.qmin, d.dq, dqinv)) - d.c_lo;
+  const long long by = to_int(floor_div(hy - d.qmin, d.dq, dqinv)) - d.c_lo;
+  if (bx < 0 || bx >= d.c_n || by < 0 || by >= d.c_n) return;
+  const C *col = reinterpret_cast<const C *>(d.inter) + ((int64_t)fb * d.W + wcol) * d.Z;
+  const bool k0 = (j == N / 2);
+  C u = C{(T)0, (T)0};
+  if (!d.fill_bkg && d.smooth) u = reinterpret_cast<const C *>(d.col_spec)[(int64_t)fb * d.W + wcol];
+  const double *sz_row = d.col_sz + (int64_t)fb * N;
+  const C *chirp = reinterpret_cast<const C *>(d.bs_chirp);
+  C a0 = C{(T)0, (T)0};
+  if (k0 && (d.fill_bkg || d.smooth))
+    a0 = C{(T)(d.avg_re * d.max_voxels * (double)N), (T)(d.avg_im * d.max_voxels * (double)N)};
+  // rows of the band, as in k_colpass_bs (>= Z); without a0, rows from Z on are zero unless
+  // smoothing without fill spreads over them
+  const bool head = (d.fill_bkg || !d.smooth) && d.Z <= GX_WAVE * CHW_NZ;
+  const int Lc = (int)min((int64_t)N, d.bs_Mc - d.bs_ck + 1);
+  C v[CHW_P];
+  auto load = [&](int q) {
+    const int z = lane + GX_WAVE * q;
+    v[q] = C{(T)0, (T)0};
+    if (z < Lc) v[q] = cmul(csub(col_input(d, col, z, k0, u, sz_row), a0), chirp[z]);
+  };
+  if (head) {
+#pragma unroll
+    for (int q = 0; q < CHW_NZ; ++q) load(q);
+    DftHead<16, CHW_NZ, C>::run(v);
+  } else {
+#pragma unroll
+    for (int q = 0; q < CHW_P; ++q) load(q);
+    DftHead<16, CHW_P, C>::run(v);
+  }
+  chirpz_wave<C>(v, lds[wave], reinterpret_cast<const C *>(d.bs_kernel_c),
+                 reinterpret_cast<const C *>(d.bs_twiddle_c), lane);
+  const int64_t cbase = (by * d.c_n + bx) * d.c_n;
+  const double val = d.q_val;
+  const int nn = (N - 1) / 2 + 1;  // fftfreq: k < nn are the non-negative frequencies
+#pragma unroll
+  for (int q = 0; q < G; ++q) {
+    const int jj = lane + GX_WAVE * q;
+    if (jj >= (int)d.bs_ck) continue;
+    const int k = (int)d.bs_clo + jj;    // signed frequency, -N/2 <= k < N - N/2
+    const int i = k + N / 2;             // fftshifted row
+    if (i < d.i_lo || i > d.i_hi) continue;
+    const int kk = k < 0 ? k + N : k;
+    const int kint = (kk < nn) ? kk : kk - N;
+    const double qz = (((double)kint * val) * 2.0) * M_PI;
+    const long long bz = to_int(floor_div(qz - d.qmin, d.dq, dqinv)) - d.c_lo;
+    if (bz < 0 || bz >= d.c_n) continue;
+    C F = cmul(v[q], chirp[k < 0 ? -k : k]);
+    if (k0 && k == 0) F = C{(T)((double)F.x + (double)a0.x * (double)N), (T)((double)F.y + (double)a0.y * (double)N)};
+    const double I = (double)cnorm(F);
+    const unsigned long long fx = (unsigned long long)llrint(I * d.bin_scale);
+    atomicAdd(&d.bin_sum[cbase + bz], fx);
+    atomicAdd(&d.bin_cnt[cbase + bz], 1);
+  }
+}
+
 template <int M, typename C>
 __global__ __launch_bounds__(GX_BLK_FFT) void k_colpass_bs(gx_frames d, int64_t f0) {
   GX_RESOLVE_AVG(d);
@@ -1631,18 +1864,42 @@ int launch_rowpass_bs_t(const gx_frames *d, int64_t f0, int64_t nf, hipStream_t 
   return check_launch("k_rowpass_bs");
 }
 
+template <typename C, int G>
+int launch_rowpass_bsw(const gx_frames *d, int64_t f0, int64_t nf, hipStream_t st) {
+  constexpr int RB = BLK / GX_WAVE;
+  const size_t lds = ((size_t)RB * CHW_BUF + (sizeof(C) == 8 ? CHW_M : 0)) * sizeof(C);  // staged rows: W <= bs_rk <= 1024
+  static bool attr_set = false;
+  if (!attr_set) {
+    GX_HIP(hipFuncSetAttribute((const void *)k_rowpass_bsw<C, G>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               160 * 1024));
+    attr_set = true;
+  }
+  k_rowpass_bsw<C, G><<<dim3((unsigned)(d->Z / RB), (unsigned)nf), BLK, lds, st>>>(*d, f0);
+  return check_launch("k_rowpass_bsw");
+}
+
+template <typename C, int G>
+int launch_colpass_bsw(const gx_frames *d, int64_t f0, int64_t nf, hipStream_t st) {
+  k_colpass_bsw<C, G><<<dim3(grid1d(d->W, BLK / GX_WAVE), (unsigned)nf), BLK, 0, st>>>(*d, f0);
+  return check_launch("k_colpass_bsw");
+}
+
 template <typename C>
 int launch_bs(const gx_frames *d, int64_t f0, int64_t nf, hipStream_t st, bool row) {
   if (row) {
     switch (d->bs_M) {
-      case 1024: return launch_rowpass_bs_t<1024, C>(d, f0, nf, st);
+      case 1024:
+        return d->bs_rk <= GX_WAVE * CHW_G ? launch_rowpass_bsw<C, CHW_G>(d, f0, nf, st)
+                                           : launch_rowpass_bsw<C, CHW_P>(d, f0, nf, st);
       case 2048: return launch_rowpass_bs_t<2048, C>(d, f0, nf, st);
       case 4096: return launch_rowpass_bs_t<4096, C>(d, f0, nf, st);
     }
   } else {
     dim3 grid((unsigned)d->W, (unsigned)nf);
     switch (d->bs_Mc) {
-      case 1024: k_colpass_bs<1024, C><<<grid, GX_BLK_FFT, 0, st>>>(*d, f0); return check_launch("k_colpass_bs");
+      case 1024:
+        return d->bs_ck <= GX_WAVE * CHW_G ? launch_colpass_bsw<C, CHW_G>(d, f0, nf, st)
+                                           : launch_colpass_bsw<C, CHW_P>(d, f0, nf, st);
       case 2048: k_colpass_bs<2048, C><<<grid, GX_BLK_FFT, 0, st>>>(*d, f0); return check_launch("k_colpass_bs");
       case 4096: k_colpass_bs<4096, C><<<grid, GX_BLK_FFT, 0, st>>>(*d, f0); return check_launch("k_colpass_bs");
     }
