@@ -558,7 +558,7 @@ __global__ __launch_bounds__(BLK) void k_adj_avg_reduce(gx_frames d, gx_adjoint 
 // adjoint of the row pass: rows of the grid's cotangent, gathered at the atoms
 // ------------------------------------------------------------------------------------
 // The gather of the gradient kernels, once `rows` holds the masked cotangent of grid rows
-// z0 .. z0 + RB (row stride N): every atom of rows z0 .. z0 + RB - 1 gathers its four
+// z0 .. z0 + RB (row stride `stride`): every atom of rows z0 .. z0 + RB - 1 gathers its four
 // nodes and writes its dL/dy', dL/dz (and, with more than GX_ADJ_ELEM_REG elements,
 // dL/df re, im) for this frame to g_part; the block's share of sum_a dL/dy'_a (fixed
 // partition of the regrouped order) goes to red, the argmin of y' to amin and, with
@@ -571,7 +571,8 @@ __device__ __forceinline__ double node_my(const gx_frames &d, const double *sy_r
 
 template <typename C>
 __device__ __forceinline__ void rowgrad_gather(const gx_frames &d, const gx_adjoint &g, const double *fp, int fb,
-                                               int rb, int nrb, int z0, int RB, int N, const C *rows, const double *ftab,
+                                               int rb, int nrb, int z0, int RB, int N, const C *rows, int stride,
+                                               const double *ftab,
                                                double *shd, int *shi, const double *mzr = nullptr,
                                                int ya = 0, int yb = 0) {
   using T = typename Real<C>::T;
@@ -617,8 +618,8 @@ __device__ __forceinline__ void rowgrad_gather(const gx_frames &d, const gx_adjo
       const double fr = ftab[2 * es[k]], fi = ftab[2 * es[k] + 1];
       double gu = 0.0, gv = 0.0, gfr = 0.0, gfi = 0.0;
       if (u0 >= 0 && vr >= 0 && vr < RB) {
-        const C *r0 = rows + vr * N + u0;
-        const C *r1 = r0 + N;
+        const C *r0 = rows + vr * stride + u0;
+        const C *r1 = r0 + stride;
         double g00r = (double)r0[0].x, g00i = (double)r0[0].y;
         double g01r = (double)r0[1].x, g01i = (double)r0[1].y;
         double g10r = (double)r1[0].x, g10i = (double)r1[0].y;
@@ -771,7 +772,7 @@ __global__ __launch_bounds__(BLK) void k_adj_rowgrad(gx_frames d, gx_adjoint g, 
   }
   __syncthreads();
 
-  rowgrad_gather<C>(d, g, fp, fb, rf.rb, nrb, z0, RB, N, rows, ftab, shd, shi, masked ? mzr : nullptr, ya, yb);
+  rowgrad_gather<C>(d, g, fp, fb, rf.rb, nrb, z0, RB, N, rows, N, ftab, shd, shi, masked ? mzr : nullptr, ya, yb);
 }
 
 // e_sum += the batch's per-frame, per-row-block dL/df sums, in two steps with fixed
@@ -1219,7 +1220,386 @@ __global__ __launch_bounds__(GX_BLK_FFT) void k_adj_rowgrad_bs(gx_frames d, gx_a
       }
   }
   __syncthreads();
-  rowgrad_gather<C>(d, g, fp, fb, blockIdx.x, gridDim.x, z0, RB, N, rows, ftab, shd, shi);
+  rowgrad_gather<C>(d, g, fp, fb, blockIdx.x, gridDim.x, z0, RB, N, rows, N, ftab, shd, shi);
+}
+
+// ------------------------------------------------------------------------------------
+// the same three passes for bands of length 1024, a row or column per wave (chirpz_wave)
+//
+// Against the block-wide forms (four points per thread, twenty block barriers a transform), one
+// evaluation of the fit geometry (N = 1048, 139,000 four-row blocks, 200,000 columns, FP32):
+// row pass 4.21 -> 2.17 ms, column adjoint 3.04 -> 1.76 ms, row gradient 9.22 -> 3.87 ms.  The
+// row and column passes issue vector instructions 65-75% of the time; the row gradient 60%, its
+// gather's LDS reads most of the rest.
+// ------------------------------------------------------------------------------------
+constexpr int CHW_RB = NWAVE;  // rows per block: one per wave
+
+// forward row pass: the block deposits the atoms of its four rows at once (each atom is read
+// by at most two blocks), then a wave transforms each row
+template <typename C, int G>
+__global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(sizeof(C) == 8 ? 4 : 2)))
+void k_adj_rowpass_bsw(gx_frames d, gx_adjoint g, int64_t f0) {
+  using T = typename Real<C>::T;
+  using AT = typename DepositAcc<C>::T;
+  using AU = typename DepositAcc<C>::U;
+  constexpr int RB = CHW_RB;
+  constexpr int ROW = 2 * CHW_BUF;  // accumulators per row: [2][1024] in the row's exchange buffer
+  static_assert(2 * sizeof(AU) == sizeof(C), "the accumulators of a row fit its exchange buffer");
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  C *bufs = reinterpret_cast<C *>(smem_raw);  // [RB][CHW_BUF]
+  AU *accs = reinterpret_cast<AU *>(smem_raw);
+  double *ftab = reinterpret_cast<double *>(bufs + RB * CHW_BUF);  // [n_elem][2]
+  C *cm = reinterpret_cast<C *>(ftab + 2 * g.n_elem);              // [1024] chirp times node mask (FP32)
+  __shared__ double rsc[RB];
+  const int lane = threadIdx.x & (GX_WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / GX_WAVE);
+  const int N = (int)d.N;
+  const int fb = blockIdx.y;
+  const double *fp = d.fparams + (f0 + fb) * GX_FP_STRIDE;
+  const int jlo = (int)fp[GX_FP_JLO], jhi = (int)fp[GX_FP_JHI];
+  const int wf = jhi - jlo + 1;
+  if (wf <= 0) return;  // block-uniform
+  const int32_t *bnd = d.idx_bounds + 4 * fb;
+  if (wf > d.W || jlo < d.bs_rlo + N / 2 || jhi > d.bs_rlo + d.bs_rk - 1 + N / 2 ||
+      (bnd[1] != INT_MIN && bnd[1] + 1 > d.bs_M - d.bs_rk)) {  // as k_adj_rowpass_bs
+    if (threadIdx.x == 0 && blockIdx.x == 0) atomicAdd(&d.status[1], 1);
+    return;
+  }
+  const C *chirp = reinterpret_cast<const C *>(d.bs_chirp);
+  const int z0 = blockIdx.x * RB, v = z0 + wave;  // Z is a multiple of 8
+  const int ylo = bnd[0], yhi = bnd[1], zlo = bnd[2], zhi = bnd[3];
+  const int ya = d.fill_bkg ? (ylo == INT_MAX ? N : ylo + 1) : 0;
+  const int yb = d.fill_bkg ? (yhi == INT_MIN ? 0 : yhi) : N;
+  const bool head = bnd[1] + 1 < GX_WAVE * CHW_NZ;  // the frame's deposits end below (block-uniform)
+  auto chirp_mask = [&](int n) {
+    C x = C{(T)0, (T)0};
+    if (n < N && n >= ya && n < yb) {
+      x = chirp[n];
+      if (d.smooth) {
+        const T m = (T)d.col_sy[(int64_t)fb * N + n];
+        x = C{x.x * m, x.y * m};
+      }
+    }
+    return x;
+  };
+  for (int i = threadIdx.x; i < 2 * g.n_elem; i += BLK) ftab[i] = g.f_table[i];
+  if constexpr (sizeof(C) == 8) {  // as k_rowpass_bsw
+#pragma unroll
+    for (int i = 0; i < CHW_M / BLK; ++i) {
+      const int n = threadIdx.x + BLK * i;
+      if (!(head && n >= GX_WAVE * CHW_NZ)) cm[n] = chirp_mask(n);
+    }
+  }
+  if (threadIdx.x < RB) rsc[threadIdx.x] = ldexp(1.0, g.row_exp[min(z0 + (int)threadIdx.x, N - 1)]);
+  {
+    int4 *p = reinterpret_cast<int4 *>(smem_raw);
+    for (int i = threadIdx.x; i < (int)(RB * CHW_BUF * sizeof(C) / 16); i += BLK) p[i] = make_int4(0, 0, 0, 0);
+  }
+  __syncthreads();
+  const double s = fp[GX_FP_SIN], c = fp[GX_FP_COS];
+  const double ymin = dkey_inv(d.ymin_key[3 * fb]);
+  const double r = d.r, rinv = 1.0 / d.r;
+  const int nmax = min(N, CHW_M);  // both nodes lie below bs_M - bs_rk + 1 <= 1024 (checked above)
+  const int a_lo = d.row_off[z0 > 0 ? z0 - 1 : 0], a_hi = d.row_off[z0 + RB];
+  for (int a = a_lo + threadIdx.x; a < a_hi; a += BLK * AU_UNROLL) {
+    double xs[AU_UNROLL], ys[AU_UNROLL], tvs[AU_UNROLL];
+    int zr[AU_UNROLL], es[AU_UNROLL];
+#pragma unroll
+    for (int k = 0; k < AU_UNROLL; ++k) {
+      const int ak = a + k * BLK;
+      const bool ok = ak < a_hi;
+      xs[k] = ok ? d.ax[ak] : 0.0;
+      ys[k] = ok ? d.ay[ak] : 0.0;
+      tvs[k] = ok ? g.afz[ak] : 0.0;
+      zr[k] = ok ? d.azrow[ak] : 0;
+      es[k] = ok ? g.aelem[ak] : 0;
+    }
+#pragma unroll
+    for (int k = 0; k < AU_UNROLL; ++k) {
+      if (a + k * BLK >= a_hi) break;
+      const int lv = zr[k] - z0;  // -1 .. RB-1
+      double tu = 0.0;
+      const int u0 = cic_u(xs[k], ys[k], s, c, ymin, r, rinv, nmax, tu);
+      if (u0 < 0) {
+        atomicAdd(&d.status[2], 1);
+        continue;
+      }
+      const double tv = tvs[k];
+      const double fr = ftab[2 * es[k]], fi = ftab[2 * es[k] + 1];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int row = lv + h;
+        if (row < 0 || row >= RB) continue;
+        const double wv = h ? tv : 1.0 - tv;
+        const double sc = rsc[row];
+        const double w0 = (wv * (1.0 - tu)) * sc, w1 = (wv * tu) * sc;  // f (w sc) = (f w) sc exactly
+        AU *ar = accs + (size_t)row * ROW;
+        atomicAdd(&ar[u0], (AU)fx_round<AT>(fr * w0));
+        atomicAdd(&ar[CHW_M + u0], (AU)fx_round<AT>(fi * w0));
+        atomicAdd(&ar[u0 + 1], (AU)fx_round<AT>(fr * w1));
+        atomicAdd(&ar[CHW_M + u0 + 1], (AU)fx_round<AT>(fi * w1));
+      }
+    }
+  }
+  __syncthreads();
+  const bool inside = !d.fill_bkg || (v >= zlo && v < zhi);
+  const bool atoms = inside && d.row_off[v + 1] > d.row_off[v > 0 ? v - 1 : 0];  // wave-uniform
+  C *fbuf = bufs + wave * CHW_BUF;
+  C x[CHW_P];
+  if (atoms) {
+    const AU *ar = accs + (size_t)wave * ROW;
+    const double inv = 1.0 / rsc[wave];
+    auto load = [&](int q) {
+      const int n = lane + GX_WAVE * q;
+      x[q] = cmul(C{(T)((double)(AT)ar[n] * inv), (T)((double)(AT)ar[CHW_M + n] * inv)},
+                  sizeof(C) == 8 ? cm[n] : chirp_mask(n));
+    };
+    if (head) {
+#pragma unroll
+      for (int q = 0; q < CHW_NZ; ++q) load(q);
+      DftHead<16, CHW_NZ, C>::run(x);
+    } else {
+#pragma unroll
+      for (int q = 0; q < CHW_P; ++q) load(q);
+      DftHead<16, CHW_P, C>::run(x);
+    }
+    wave_sync();
+    chirpz_wave<C>(x, fbuf, reinterpret_cast<const C *>(d.bs_kernel), reinterpret_cast<const C *>(d.bs_twiddle), lane);
+    wave_sync();
+  }
+  // the band, staged in the wave's buffer
+  const bool dense = d.fill_bkg || d.smooth;
+  const double avv_re = d.avg_re * d.max_voxels, avv_im = d.avg_im * d.max_voxels;
+  const double mz = d.smooth ? d.col_sz[(int64_t)fb * N + v] : 1.0;
+  const C *spec = reinterpret_cast<const C *>(d.col_spec) + (int64_t)fb * d.W;
+#pragma unroll
+  for (int q = 0; q < G; ++q) {
+    const int j = lane + GX_WAVE * q;
+    if (j >= (int)d.bs_rk) continue;
+    const int k = (int)d.bs_rlo + j;  // signed frequency
+    const int w = k + N / 2 - jlo;    // fftshifted column within the frame's band
+    if (w < 0 || w >= wf) continue;
+    C o = C{(T)0, (T)0};
+    if (atoms) o = cmul(x[q], chirp[k < 0 ? -k : k]);
+    if (!inside) {
+      o = (k == 0) ? C{(T)(avv_re * (double)N), (T)(avv_im * (double)N)} : C{(T)0, (T)0};
+    } else if (dense) {
+      const C u = spec[w];
+      double ore = mz * ((double)o.x + (double)u.x);
+      double oim = mz * ((double)o.y + (double)u.y);
+      if (d.smooth && k == 0) {
+        ore = ore + avv_re * (double)N;
+        oim = oim + avv_im * (double)N;
+      }
+      o = C{(T)ore, (T)oim};
+    }
+    fbuf[w] = o;
+  }
+  __syncthreads();
+  C *out = reinterpret_cast<C *>(d.inter) + (int64_t)fb * d.W * d.Z + z0;
+  for (int idx = threadIdx.x; idx < wf * RB; idx += BLK) {
+    const int w = idx / RB, q = idx - w * RB;
+    out[(int64_t)w * d.Z + q] = bufs[q * CHW_BUF + w];
+  }
+}
+
+// adjoint of the column pass (in place on d.inter): as k_adj_colpass_bs, a wave per kept
+// column; F as k_colpass_bsw forms it (the k = 0 column's constant taken out of the transform)
+template <typename C, int G>
+__global__ __launch_bounds__(BLK) void k_adj_colpass_bsw(gx_frames d, gx_adjoint g, int64_t f0) {
+  using T = typename Real<C>::T;
+  __shared__ C lds[NWAVE][CHW_BUF];
+  const int N = (int)d.N;
+  const int lane = threadIdx.x & (GX_WAVE - 1);
+  const int wave = threadIdx.x / GX_WAVE;
+  const int fb = blockIdx.y;
+  const double *fp = d.fparams + (f0 + fb) * GX_FP_STRIDE;
+  const int jlo = (int)fp[GX_FP_JLO], jhi = (int)fp[GX_FP_JHI];
+  if (blockIdx.x == 0 && threadIdx.x == 0) g.amin[fb] = INT_MAX;  // argmin slot of the gradient gather
+  const int wcol = blockIdx.x * NWAVE + wave;
+  if (wcol > jhi - jlo || wcol >= d.W) return;  // wave-uniform; no block barrier below
+  const bool dense = d.fill_bkg || d.smooth;
+  double2 *apart = reinterpret_cast<double2 *>(g.avg_part);
+  C *col = reinterpret_cast<C *>(d.inter) + ((int64_t)fb * d.W + wcol) * d.Z;
+  const int j = jlo + wcol;
+  const double hx = (j == N - 1) ? fp[GX_FP_HX_STOP] : (double)j * fp[GX_FP_HX_STEP] + fp[GX_FP_HX_START];
+  const double hy = (j == N - 1) ? fp[GX_FP_HY_STOP] : (double)j * fp[GX_FP_HY_STEP] + fp[GX_FP_HY_START];
+  const double dqinv = 1.0 / d.dq;
+  const long long bx = to_int(floor_div(hx - d.qmin, d.dq, dqinv)) - d.c_lo;
+  const long long by = to_int(floor_div(hy - d.qmin, d.dq, dqinv)) - d.c_lo;
+  if (bx < 0 || bx >= d.c_n || by < 0 || by >= d.c_n) {  // never binned: zero cotangent
+    for (int z = lane; z < d.Z; z += GX_WAVE) col[z] = C{(T)0, (T)0};
+    if (dense && lane == 0) apart[(int64_t)fb * d.W + wcol] = make_double2(0.0, 0.0);
+    return;
+  }
+  const bool k0 = (j == N / 2);
+  C u = C{(T)0, (T)0};
+  if (!d.fill_bkg && d.smooth) u = reinterpret_cast<const C *>(d.col_spec)[(int64_t)fb * d.W + wcol];
+  const double *sz_row = d.col_sz + (int64_t)fb * N;
+  const C *chirp = reinterpret_cast<const C *>(d.bs_chirp);
+  const C *tw = reinterpret_cast<const C *>(d.bs_twiddle_c);
+  C a0 = C{(T)0, (T)0};
+  if (k0 && dense)
+    a0 = C{(T)(d.avg_re * d.max_voxels * (double)N), (T)(d.avg_im * d.max_voxels * (double)N)};
+  const bool head = (d.fill_bkg || !d.smooth) && d.Z <= GX_WAVE * CHW_NZ;  // as k_colpass_bsw
+  const int Lc = (int)min((int64_t)N, d.bs_Mc - d.bs_ck + 1);
+  C v[CHW_P];
+  auto load = [&](int q) {
+    const int z = lane + GX_WAVE * q;
+    v[q] = C{(T)0, (T)0};
+    if (z < Lc) v[q] = cmul(csub(col_input(d, (const C *)col, z, k0, u, sz_row), a0), chirp[z]);
+  };
+  if (head) {
+#pragma unroll
+    for (int q = 0; q < CHW_NZ; ++q) load(q);
+    DftHead<16, CHW_NZ, C>::run(v);
+  } else {
+#pragma unroll
+    for (int q = 0; q < CHW_P; ++q) load(q);
+    DftHead<16, CHW_P, C>::run(v);
+  }
+  chirpz_wave<C>(v, lds[wave], reinterpret_cast<const C *>(d.bs_kernel_c), tw, lane);
+  const int64_t cbase = (by * d.c_n + bx) * d.c_n;
+  const double val = d.q_val;
+  const int nn = (N - 1) / 2 + 1;  // fftfreq: k < nn are the non-negative frequencies
+  const double2 *zhat = reinterpret_cast<const double2 *>(g.avg_spec) + (int64_t)fb * (N + d.W);
+  double are = 0.0, aim = 0.0, dc_re = 0.0, dc_im = 0.0;
+#pragma unroll
+  for (int q = 0; q < G; ++q) {
+    const int jj = lane + GX_WAVE * q;
+    C a = C{(T)0, (T)0};
+    if (jj < (int)d.bs_ck) {
+      const int k = (int)d.bs_clo + jj;  // signed frequency
+      const int i = k + N / 2;           // fftshifted row
+      const int kk = k < 0 ? k + N : k;  // natural index
+      if (i >= d.i_lo && i <= d.i_hi) {
+        const int kint = (kk < nn) ? kk : kk - N;
+        const double qz = (((double)kint * val) * 2.0) * M_PI;
+        const long long bz = to_int(floor_div(qz - d.qmin, d.dq, dqinv)) - d.c_lo;
+        if (bz >= 0 && bz < d.c_n) {
+          const C ck = chirp[k < 0 ? -k : k];
+          const double gI = 2.0 * g.g_bins[cbase + bz];
+          C F = cmul(v[q], ck);
+          if (k0 && k == 0)
+            F = C{(T)((double)F.x + (double)a0.x * (double)N), (T)((double)F.y + (double)a0.y * (double)N)};
+          const double gr = gI * (double)F.x, gi = gI * (double)F.y;
+          if (dense) {
+            const double2 zh = zhat[kk];
+            are += gr * zh.x + gi * zh.y;
+            aim += gi * zh.x - gr * zh.y;
+            if (kk == 0) {
+              dc_re = gr;
+              dc_im = gi;
+            }
+          }
+          a = cmul(C{(T)gr, (T)(-gi)}, ck);  // conj(dL/dF) c[|k|]
+        }
+      }
+    }
+    v[q] = a;
+  }
+  if (dense) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      are += __shfl_xor(are, off, GX_WAVE);
+      aim += __shfl_xor(aim, off, GX_WAVE);
+      dc_re += __shfl_xor(dc_re, off, GX_WAVE);  // one lane's value, the rest zeros
+      dc_im += __shfl_xor(dc_im, off, GX_WAVE);
+    }
+    if (lane == 0) {
+      const double2 yh = zhat[N + wcol];
+      double pre = are * yh.x + aim * yh.y, pim = aim * yh.x - are * yh.y;
+      if (k0) {
+        const double c0 = d.max_voxels * (double)N * (double)N;
+        pre = pre + c0 * dc_re;
+        pim = pim + c0 * dc_im;
+      }
+      apart[(int64_t)fb * d.W + wcol] = make_double2(pre, pim);
+    }
+  }
+  DftHead<16, G, C>::run(v);
+  wave_sync();
+  chirpz_wave<C>(v, lds[wave], reinterpret_cast<const C *>(g.bs_kernel_adj_c), tw, lane);
+  // dL/dx[z] = conj(c[z] y[z])
+#pragma unroll
+  for (int q = 0; q < CHW_P; ++q) {
+    const int z = lane + GX_WAVE * q;
+    if (z < d.Z) col[z] = cconj(cmul(v[q], chirp[z]));
+  }
+}
+
+// adjoint of the row pass: the block's four rows (the last the halo row), one per wave, back
+// to grid points, conjugated and unmasked; then the gather, which applies the node mask
+template <typename C, int G>
+__global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(sizeof(C) == 8 ? 4 : 2)))
+void k_adj_rowgrad_bsw(gx_frames d, gx_adjoint g, int64_t f0) {
+  using T = typename Real<C>::T;
+  constexpr int H = BS_GRAD_H, RB = H - 1;
+  static_assert(H == NWAVE, "one row per wave");
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  C *rows = reinterpret_cast<C *>(smem_raw);  // [H][CHW_BUF] exchange buffers, then the rows' cotangent
+  C *stage = rows;                            // [W][H], consumed before the exchanges (wf <= bs_rk <= 1024)
+  double *ftab = reinterpret_cast<double *>(rows + H * CHW_BUF);  // [n_elem][2]
+  __shared__ double mzr[H];  // z part of the node mask of the block's rows
+  __shared__ double shd[NWAVE];
+  __shared__ int shi[NWAVE];
+  const int N = (int)d.N;
+  const int lane = threadIdx.x & (GX_WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / GX_WAVE);
+  const int fb = blockIdx.y;
+  const double *fp = d.fparams + (f0 + fb) * GX_FP_STRIDE;
+  const int jlo = (int)fp[GX_FP_JLO], jhi = (int)fp[GX_FP_JHI];
+  const int wf = max(0, min(jhi - jlo + 1, (int)min(d.W, d.bs_rk)));
+  const int z0 = blockIdx.x * RB;
+  const int32_t *bnd = d.idx_bounds + 4 * fb;
+  if (bnd[1] != INT_MIN && bnd[1] + 1 > d.bs_M - d.bs_rk) {  // as k_adj_rowgrad_bs
+    if (threadIdx.x == 0 && blockIdx.x == 0) atomicAdd(&d.status[1], 1);
+    return;
+  }
+  for (int i = threadIdx.x; i < 2 * g.n_elem; i += BLK) ftab[i] = g.f_table[i];
+  const int ylo = bnd[0], yhi = bnd[1], zlo = bnd[2], zhi = bnd[3];
+  const int ya = d.fill_bkg ? (ylo == INT_MAX ? N : ylo + 1) : 0;
+  const int yb = d.fill_bkg ? (yhi == INT_MIN ? 0 : yhi) : N;
+  const bool masked = d.fill_bkg || d.smooth;
+  if (threadIdx.x < H) {
+    const int v = z0 + threadIdx.x;
+    double mzv = 1.0;
+    if (d.fill_bkg && !(v >= zlo && v < zhi)) mzv = 0.0;
+    if (d.smooth && v < N) mzv = mzv * d.col_sz[(int64_t)fb * N + v];
+    mzr[threadIdx.x] = mzv;
+  }
+  const C *src = reinterpret_cast<const C *>(d.inter) + (int64_t)fb * d.W * d.Z;
+  for (int idx = threadIdx.x; idx < wf * H; idx += BLK) {
+    const int w = idx / H, q = idx - w * H;
+    const int v = z0 + q;
+    stage[idx] = (v < d.Z) ? src[(int64_t)w * d.Z + v] : C{(T)0, (T)0};
+  }
+  __syncthreads();
+  const C *chirp = reinterpret_cast<const C *>(d.bs_chirp);
+  C x[CHW_P];
+#pragma unroll
+  for (int q = 0; q < G; ++q) {
+    const int jj = lane + GX_WAVE * q;
+    x[q] = C{(T)0, (T)0};
+    if (jj < (int)d.bs_rk) {
+      const int k = (int)d.bs_rlo + jj;
+      const int w = k + N / 2 - jlo;
+      if (w >= 0 && w < wf) x[q] = cmul(cconj(stage[w * H + wave]), chirp[k < 0 ? -k : k]);
+    }
+  }
+  DftHead<16, G, C>::run(x);
+  __syncthreads();
+  C *buf = rows + wave * CHW_BUF;
+  chirpz_wave<C>(x, buf, reinterpret_cast<const C *>(g.bs_kernel_adj), reinterpret_cast<const C *>(d.bs_twiddle), lane);
+  wave_sync();
+#pragma unroll
+  for (int q = 0; q < CHW_P; ++q) {
+    const int o = lane + GX_WAVE * q;
+    if (o < N) buf[o] = cconj(cmul(x[q], chirp[o]));
+  }
+  __syncthreads();
+  rowgrad_gather<C>(d, g, fp, fb, blockIdx.x, gridDim.x, z0, RB, N, rows, CHW_BUF, ftab, shd, shi,
+                    masked ? mzr : nullptr, ya, yb);
 }
 
 // ------------------------------------------------------------------------------------
@@ -1542,11 +1922,39 @@ int launch_adj_bs_t(Op op, const gx_frames *d, const gx_adjoint *g, int64_t f0, 
   return check_launch("k_adj_rowgrad_bs");
 }
 
+// the passes of length 1024 (a row or column per wave); G: 64-value groups of the band
+template <typename C, int G>
+int launch_adj_bsw(Op op, const gx_frames *d, const gx_adjoint *g, int64_t f0, int64_t nf, hipStream_t st) {
+  if (op == OP_COLPASS) {
+    k_adj_colpass_bsw<C, G><<<dim3(grid1d(d->W, NWAVE), (unsigned)nf), BLK, 0, st>>>(*d, *g, f0);
+    return check_launch("k_adj_colpass_bsw");
+  }
+  static bool attr_set = false;
+  if (!attr_set) {
+    GX_HIP(hipFuncSetAttribute((const void *)k_adj_rowpass_bsw<C, G>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               150 * 1024));
+    GX_HIP(hipFuncSetAttribute((const void *)k_adj_rowgrad_bsw<C, G>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               150 * 1024));
+    attr_set = true;
+  }
+  const size_t lds = (size_t)NWAVE * CHW_BUF * sizeof(C) + (size_t)g->n_elem * 16;
+  if (op == OP_ROWPASS) {
+    const size_t cm = sizeof(C) == 8 ? CHW_M * sizeof(C) : 0;
+    k_adj_rowpass_bsw<C, G><<<dim3((unsigned)(d->Z / CHW_RB), (unsigned)nf), BLK, lds + cm, st>>>(*d, *g, f0);
+    return check_launch("k_adj_rowpass_bsw");
+  }
+  k_adj_rowgrad_bsw<C, G><<<dim3((unsigned)rowgrad_blocks(d), (unsigned)nf), BLK, lds, st>>>(*d, *g, f0);
+  return check_launch("k_adj_rowgrad_bsw");
+}
+
 template <typename C>
 int dispatch_bs_c(Op op, const gx_frames *d, const gx_adjoint *g, int64_t f0, int64_t nf, hipStream_t st) {
   const int64_t M = (op == OP_COLPASS) ? d->bs_Mc : d->bs_M;
   switch (M) {
-    case 1024: return launch_adj_bs_t<1024, C>(op, d, g, f0, nf, st);
+    case 1024:
+      return (op == OP_COLPASS ? d->bs_ck : d->bs_rk) <= GX_WAVE * CHW_G
+                 ? launch_adj_bsw<C, CHW_G>(op, d, g, f0, nf, st)
+                 : launch_adj_bsw<C, CHW_P>(op, d, g, f0, nf, st);
     case 2048: return launch_adj_bs_t<2048, C>(op, d, g, f0, nf, st);
     case 4096: return launch_adj_bs_t<4096, C>(op, d, g, f0, nf, st);
     default: return set_error(GX_ERR_UNSUPPORTED, "chirp-z transform length %lld", (long long)M);
