@@ -696,13 +696,19 @@ __global__ __launch_bounds__(BLK) void k_det_fin_adj(const double *__restrict__ 
 
 // One block: fx_scale = 2^(61 - floor(log2 B)) with B = mult * sum(part) * sum_o |w_o|,
 // a bound on every |dL/d iq| and on every partial sum of the scatter below (mult
-// = 4 covers the mirror, whose outputs add at most four inputs).
-__global__ __launch_bounds__(BLK) void k_det_scale(const double *__restrict__ part, int64_t n_part, double mult,
-                                                   const double *w, int64_t n_orient, double *fx_scale) {
+// = 4 covers the mirror, whose outputs add at most four inputs).  uniform_w (may overlap
+// part, not NULL for the mapped adjoint): 1 if every weight equals the first, else 0.
+__global__ __launch_bounds__(BLK) void k_det_scale(const double *part, int64_t n_part, double mult,
+                                                   const double *w, int64_t n_orient, double *fx_scale,
+                                                   double *uniform_w) {
   __shared__ double sh[2][BLK / GX_WAVE];
   double a = 0.0, b = 0.0;
+  bool other = false;
   for (int64_t i = threadIdx.x; i < n_part; i += BLK) a += part[i];
-  for (int64_t o = threadIdx.x; o < n_orient; o += BLK) b += fabs(w[o]);
+  for (int64_t o = threadIdx.x; o < n_orient; o += BLK) {
+    b += fabs(w[o]);
+    other |= !(w[o] == w[0]);
+  }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
     a += __shfl_xor(a, off, GX_WAVE);
@@ -713,8 +719,9 @@ __global__ __launch_bounds__(BLK) void k_det_scale(const double *__restrict__ pa
     sh[0][wv] = a;
     sh[1][wv] = b;
   }
-  __syncthreads();
+  const bool mixed = __syncthreads_or(other);
   if (threadIdx.x == 0) {
+    if (uniform_w) uniform_w[0] = mixed ? 0.0 : 1.0;
     double A = 0.0, B = 0.0;
     for (int i = 0; i < BLK / GX_WAVE; ++i) {
       A += sh[0][i];
@@ -913,67 +920,122 @@ __global__ __launch_bounds__(BLK) void k_det_adj_prefix(const double *__restrict
   if (p < npx) S[p] = t;
 }
 
-// dL/d iq per voxel from the transpose map, balanced over runs: a wave takes
-// MAP_UNROLL chunks of 64 consecutive runs of the voxel-sorted map (every load of the
-// chunks is issued before the first use); each lane sums its run's fixed-point terms
-// g[p] w[o] (one per pixel, rounded as the scatter path rounds them: from the prefix
-// table when w[o] is the first orientation's weight, the usual case of uniform weights,
-// else pixel by pixel), the wave sums runs of equal voxel with a segmented scan across
-// the lanes, and the last lane of each segment adds its total to g_fx[voxel] with an
-// integer atomic.  Integer sums are exact, so the result does not depend on the order.
-// g_fx starts at zero.
-constexpr int MAP_UNROLL = 4;
+// dL/d iq per voxel from the transpose map, balanced over runs: a wave takes chunks of
+// 64 MAP_RPL consecutive runs of the voxel-sorted map, MAP_RPL neighbouring ones per lane
+// (loaded together).  Each run's sum of fixed-point terms g[p] w[o] (one per pixel, rounded as
+// the scatter path rounds them) comes from the prefix table when w[o] is the first
+// orientation's weight, the usual case of uniform weights, else pixel by pixel; a segment of
+// equal voxel sums to the difference of two prefixes over the chunk's runs, and its last run
+// adds it to g_fx[voxel] with an integer atomic.  Integer sums are exact (also modulo 2^64 in
+// the chunk's prefix), so the result does not depend on the order.  g_fx starts at zero.
+//
+// Bound by the table's gathers (two per run, mostly of one line: 1,470 M line lookups and 245 M
+// L2 requests for the 848 M runs of 16,380 orientations of 250^2 pixels): 6.30 -> 3.07 ms
+// against one run per lane, a segmented scan of 18 lane exchanges per 64 runs and a weight
+// gathered per run.  Single pixels' terms in a table of their own halve the lookups but lose
+// the shared lines (3.6 ms).
+constexpr int MAP_RPL = 4;
+
+// inclusive prefix sum over the wave's lanes, modulo 2^64 (row shifts, then the row totals)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned long long dpp_add(unsigned long long x) {
+  const unsigned lo = __builtin_amdgcn_update_dpp(0u, (unsigned)x, CTRL, ROWS, 0xf, false);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0u, (unsigned)(x >> 32), CTRL, ROWS, 0xf, false);
+  return x + (((unsigned long long)hi << 32) | lo);
+}
+__device__ __forceinline__ unsigned long long wave_prefix(unsigned long long x) {
+  x = dpp_add<0x111, 0xf>(x);  // row_shr:1, 2, 4, 8
+  x = dpp_add<0x112, 0xf>(x);
+  x = dpp_add<0x114, 0xf>(x);
+  x = dpp_add<0x118, 0xf>(x);
+  x = dpp_add<0x142, 0xa>(x);  // row_bcast:15 into rows 1, 3; row_bcast:31 into rows 2, 3
+  x = dpp_add<0x143, 0xc>(x);
+  return x;
+}
 
 __global__ __launch_bounds__(BLK) void k_det_adj_map(gx_detector d, const double *__restrict__ g,
                                                      const long long *__restrict__ S, const double *fx_scale,
-                                                     const int32_t *__restrict__ run_voxel,
+                                                     const double *uniform_w, const int32_t *__restrict__ run_voxel,
                                                      const uint32_t *__restrict__ runs,
                                                      const uint8_t *__restrict__ run_len, int64_t n_runs,
                                                      unsigned long long *g_fx, int pbits) {
-  constexpr int SPAN = MAP_UNROLL * GX_WAVE;  // runs per wave and step
+  constexpr int R = MAP_RPL, SPAN = R * GX_WAVE;  // runs per wave and step
   const int lane = threadIdx.x & (GX_WAVE - 1);
-  const double sc = fx_scale[0], w0 = d.orient_w[0];
+  const bool uniform = uniform_w[0] != 0.0;  // every orientation has the first one's weight
   const uint32_t pmask = (pbits >= 32) ? 0xffffffffu : ((1u << pbits) - 1u);
   const int64_t wave0 = (blockIdx.x * (int64_t)BLK + threadIdx.x) / GX_WAVE;
   const int64_t n_waves = (int64_t)gridDim.x * (BLK / GX_WAVE);
   for (int64_t base = wave0 * SPAN; base < n_runs; base += n_waves * SPAN) {
-    int v[MAP_UNROLL], len[MAP_UNROLL];
-    uint32_t id[MAP_UNROLL];
+    int v[R];
+    uint32_t id[R];
+    uint8_t len[R];
+    const int64_t k0 = base + lane * R;
+    if (base + SPAN <= n_runs) {
+      __builtin_memcpy(v, run_voxel + k0, sizeof(v));
+      __builtin_memcpy(id, runs + k0, sizeof(id));
+      __builtin_memcpy(len, run_len + k0, sizeof(len));
+    } else {
 #pragma unroll
-    for (int u = 0; u < MAP_UNROLL; ++u) {
-      const int64_t k = base + u * GX_WAVE + lane;
-      v[u] = -1;
-      id[u] = 0u;
-      len[u] = 0;
-      if (k < n_runs) {
-        v[u] = run_voxel[k];
-        id[u] = runs[k];
-        len[u] = run_len[k];
+      for (int i = 0; i < R; ++i) {
+        const bool ok = k0 + i < n_runs;
+        v[i] = ok ? run_voxel[k0 + i] : -1;
+        id[i] = ok ? runs[k0 + i] : 0u;
+        len[i] = ok ? run_len[k0 + i] : (uint8_t)0;
       }
     }
+    unsigned long long c[R];  // prefix sums of the lane's runs
+    if (uniform) {
+      long long hi[R], lo[R];
 #pragma unroll
-    for (int u = 0; u < MAP_UNROLL; ++u) {
-      long long t = 0;
-      if (v[u] >= 0) {
-        const uint32_t p = id[u] & pmask;
-        const double w = d.orient_w[id[u] >> pbits];
-        if (w == w0) {
-          long long lo = 0;
-          if (p & (GX_WAVE - 1)) lo = S[p - 1];
-          t = S[p + len[u] - 1] - lo;
-        } else {
-          for (int j = 0; j < len[u]; ++j) t += llrint((g[p + j] * w) * sc);
+      for (int i = 0; i < R; ++i) {
+        const uint32_t p = id[i] & pmask;
+        hi[i] = S[len[i] ? p + len[i] - 1 : 0];
+        lo[i] = S[p ? p - 1 : 0];
+      }
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        const long long t = hi[i] - (((id[i] & pmask) & (GX_WAVE - 1)) ? lo[i] : 0);
+        c[i] = (i ? c[i - 1] : 0ull) + (unsigned long long)(v[i] >= 0 ? t : 0);
+      }
+    } else {
+      const double sc = fx_scale[0], w0 = d.orient_w[0];
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        long long t = 0;
+        if (v[i] >= 0) {
+          const uint32_t p = id[i] & pmask;
+          const double w = d.orient_w[id[i] >> pbits];
+          if (w == w0) {
+            t = S[p + len[i] - 1] - ((p & (GX_WAVE - 1)) ? S[p - 1] : 0);
+          } else {
+            for (int j = 0; j < len[i]; ++j) t += llrint((g[p + j] * w) * sc);
+          }
         }
+        c[i] = (i ? c[i - 1] : 0ull) + (unsigned long long)t;
       }
-      // inclusive scan within segments of equal voxel (contiguous: the map is voxel-sorted)
+    }
+    const int vp = __builtin_amdgcn_update_dpp(-2, v[R - 1], 0x138, 0xf, 0xf, false);  // wave_shr:1
+    const int vn = __builtin_amdgcn_update_dpp(-2, v[0], 0x130, 0xf, 0xf, false);      // wave_shl:1
+    // X: sum of the lanes before; start: the chunk's sum before the segment of run i
+    const unsigned long long X = wave_prefix(c[R - 1]) - c[R - 1];
+    unsigned long long last = 0;  // before the last segment that begins in this lane
+    bool any = false;
 #pragma unroll
-      for (int o = 1; o < GX_WAVE; o <<= 1) {
-        const long long tu = __shfl_up(t, o, GX_WAVE);
-        const int vu = __shfl_up(v[u], o, GX_WAVE);
-        if (lane >= o && vu == v[u]) t += tu;
+    for (int i = 0; i < R; ++i)
+      if (v[i] != (i ? v[i - 1] : vp)) {
+        any = true;
+        last = X + (i ? c[i - 1] : 0ull);
       }
-      const int vn = __shfl_down(v[u], 1, GX_WAVE);
-      if (v[u] >= 0 && (lane == GX_WAVE - 1 || vn != v[u])) atomicAdd(&g_fx[v[u]], (unsigned long long)t);
+    const unsigned long long heads = __ballot(any);
+    // the segment that runs on from an earlier lane began in the nearest one with a head
+    // (lane 0 has one: its first run begins a segment)
+    int src = lane;
+    if (v[0] == vp) src = GX_WAVE - 1 - __builtin_clzll(heads & ((1ull << lane) - 1ull));
+    unsigned long long start = __shfl(last, src, GX_WAVE);
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      if (v[i] != (i ? v[i - 1] : vp)) start = X + (i ? c[i - 1] : 0ull);
+      if (v[i] >= 0 && v[i] != (i < R - 1 ? v[i + 1] : vn)) atomicAdd(&g_fx[v[i]], (X + c[i]) - start);
     }
   }
 }
@@ -1421,13 +1483,13 @@ int gx_detector_adjoint_mapped(const gx_detector *d, const double *g_out, int64_
   else
     g_raw = t;
   k_det_scale<<<1, BLK, 0, st>>>(part, nblk, (flags & GX_FIN_MIRROR) ? 4.0 : 1.0, d->orient_w, d->n_orient,
-                                 fx_scale);
+                                 fx_scale, part);
   k_det_adj_prefix<<<nblk, BLK, 0, st>>>(g_raw, d->orient_w, fx_scale, npx, S);
   const int64_t nv = d->cy * d->cx * d->cz;
   const unsigned gz = grid1d(nv, BLK);
   k_zero_u64<<<gz > 8192 ? 8192 : gz, BLK, 0, st>>>(g_fx, nv);
-  const unsigned gp = grid1d(n_runs, BLK * MAP_UNROLL);  // a wave per 64 MAP_UNROLL runs, grid-strided
-  k_det_adj_map<<<gp > 65536 ? 65536 : gp, BLK, 0, st>>>(*d, g_raw, S, fx_scale, run_voxel, runs, run_len, n_runs,
+  const unsigned gp = grid1d(n_runs, BLK * MAP_RPL);  // a wave per 64 MAP_RPL runs, grid-strided
+  k_det_adj_map<<<gp > 65536 ? 65536 : gp, BLK, 0, st>>>(*d, g_raw, S, fx_scale, part, run_voxel, runs, run_len, n_runs,
                                                          g_fx, map_pixel_bits(npx));
   return check_launch("gx_detector_adjoint_mapped");
 }
@@ -1460,7 +1522,7 @@ int gx_detector_adjoint(const gx_detector *d, const double *g_out, int64_t flags
   unsigned gz = grid1d(nv * n_rep, BLK);
   k_zero_u64<<<gz > 4096 ? 4096 : gz, BLK, 0, st>>>(g_fx, nv * n_rep);
   k_det_scale<<<1, BLK, 0, st>>>(part, nblk, (flags & GX_FIN_MIRROR) ? 4.0 : 1.0, d->orient_w, d->n_orient,
-                                 fx_scale);
+                                 fx_scale, nullptr);
   k_det_adj<<<nblk, BLK, orient_flags_lds(d), st>>>(*d, g_raw, fx_scale, g_fx, n_rep);
   return check_launch("gx_detector_adjoint");
 }
