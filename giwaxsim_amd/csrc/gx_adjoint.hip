@@ -1082,7 +1082,8 @@ __global__ __launch_bounds__(GX_BLK_FFT) void k_adj_colpass_bs(gx_frames d, gx_a
 }
 
 // FFT(Pz) at the column band and FFT(Py) on the kept columns by direct FP64 DFTs (as
-// k_adj_avg_spectra for power-of-two edges), grid (nf, 2)
+// k_adj_avg_spectra for power-of-two edges; dft_band_pair: 892 frames at N = 1048, 478 -> 57 us),
+// grid (nf, 2)
 __global__ __launch_bounds__(BLK) void k_adj_avg_spectra_dft(gx_frames d, gx_adjoint g, int64_t f0) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   double *p = reinterpret_cast<double *>(smem_raw);  // [N]
@@ -1109,31 +1110,23 @@ __global__ __launch_bounds__(BLK) void k_adj_avg_spectra_dft(gx_frames d, gx_adj
     }
     p[i] = v;
   }
+  for (int i = N + threadIdx.x; i < dft_pad(N); i += BLK) p[i] = 0.0;
   __syncthreads();
   const double2 *tw = reinterpret_cast<const double2 *>(d.twiddle64);
   double2 *out = reinterpret_cast<double2 *>(g.avg_spec) + (int64_t)fb * (N + d.W);
-  const int n_out = along_y ? wf : (int)d.bs_ck;
-  for (int o = threadIdx.x; o < n_out; o += BLK) {
-    int k;  // natural frequency index
-    if (along_y) {
-      k = (jlo + o + N - N / 2) % N;
-    } else {
-      const int ks = (int)d.bs_clo + o;
-      k = ks < 0 ? ks + N : ks;
-    }
-    double re = 0.0, im = 0.0;
-    int m = 0;
-    for (int i = 0; i < N; ++i) {
-      const double2 t = tw[m];
-      re = fma(p[i], t.x, re);
-      im = fma(p[i], t.y, im);
-      m += k;
-      if (m >= N) m -= N;
-    }
-    if (along_y)
-      out[N + o] = make_double2(re, im);
-    else
-      out[k] = make_double2(re, im);
+  // signed frequencies klo .. khi: the kept columns in order, the column band at natural index
+  const int klo = along_y ? jlo - N / 2 : (int)d.bs_clo;
+  const int khi = klo + (along_y ? wf : (int)d.bs_ck) - 1;
+  auto put = [&](int k, double2 x) {
+    if (k < klo || k > khi) return;
+    out[along_y ? N + (k - klo) : (k < 0 ? k + N : k)] = x;
+  };
+  const int k0 = klo > 0 ? klo : khi < 0 ? -khi : 0, k1 = max(-klo, khi);
+  for (int k = k0 + threadIdx.x; k <= k1; k += BLK) {
+    double2 xp, xm;
+    dft_band_pair<false>(p, N, tw, k, xp, xm);
+    put(k, xp);
+    if (k > 0) put(-k, xm);
   }
 }
 
@@ -1963,7 +1956,7 @@ int dispatch_bs_c(Op op, const gx_frames *d, const gx_adjoint *g, int64_t f0, in
 
 int dispatch_bs(Op op, const gx_frames *d, const gx_adjoint *g, int64_t f0, int64_t nf, hipStream_t st) {
   if (op == OP_AVGSPEC) {
-    k_adj_avg_spectra_dft<<<dim3((unsigned)nf, 2), BLK, (size_t)d->N * sizeof(double), st>>>(*d, *g, f0);
+    k_adj_avg_spectra_dft<<<dim3((unsigned)nf, 2), BLK, (size_t)dft_pad((int)d->N) * sizeof(double), st>>>(*d, *g, f0);
     return check_launch("k_adj_avg_spectra_dft");
   }
   if (d->fft_f64) return dispatch_bs_c<double2>(op, d, g, f0, nf, st);

@@ -844,4 +844,58 @@ __device__ __forceinline__ double f0_weight(const double *aff, double q2, double
   return fn * fn;
 }
 
+// ------------------------------------------------------------------------------------
+// Direct FP64 DFT of a short band of any edge N: X[k] and X[-k] of the profile u[0 .. N - 1]
+// (real, or complex as pairs), which the caller has put in LDS, zero-padded to a multiple of
+// DFT_PH.  With y = DFT_PH s + j the twiddle exp(-2 pi i k y / N) splits into one of s, taken
+// from the table once per DFT_PH inputs, and one of j, applied to DFT_PH partial sums at the end;
+// the two frequencies share every product.  0 <= k < N.
+// ------------------------------------------------------------------------------------
+constexpr int DFT_PH = 8;
+constexpr int dft_pad(int N) { return (N + DFT_PH - 1) / DFT_PH * DFT_PH; }
+
+template <bool CPLX>
+__device__ __forceinline__ void dft_band_pair(const double *u, int N, const double2 *__restrict__ tw, int k,
+                                              double2 &xp, double2 &xm) {
+  double a[DFT_PH], b[DFT_PH], c[DFT_PH], e[DFT_PH];  // sums of ux tx, uy ty, ux ty, uy tx
+#pragma unroll
+  for (int j = 0; j < DFT_PH; ++j) a[j] = b[j] = c[j] = e[j] = 0.0;
+  const int step = (int)(((int64_t)k * DFT_PH) % N);
+  int m = 0;
+  double2 t = tw[0];
+  for (int y = 0; y < N; y += DFT_PH) {
+    m += step;
+    if (m >= N) m -= N;
+    const double2 tn = tw[m];  // of the next step
+#pragma unroll
+    for (int j = 0; j < DFT_PH; ++j) {
+      if constexpr (CPLX) {
+        const double2 x = reinterpret_cast<const double2 *>(u)[y + j];
+        a[j] = fma(x.x, t.x, a[j]);
+        b[j] = fma(x.y, t.y, b[j]);
+        c[j] = fma(x.x, t.y, c[j]);
+        e[j] = fma(x.y, t.x, e[j]);
+      } else {
+        a[j] = fma(u[y + j], t.x, a[j]);
+        c[j] = fma(u[y + j], t.y, c[j]);
+      }
+    }
+    t = tn;
+  }
+  xp = xm = make_double2(0.0, 0.0);
+  m = 0;
+#pragma unroll
+  for (int j = 0; j < DFT_PH; ++j) {
+    const double2 w = tw[m];
+    const double pr = a[j] - b[j], pi = c[j] + e[j];  // of k
+    const double qr = a[j] + b[j], qi = e[j] - c[j];  // of -k
+    xp.x = fma(pr, w.x, fma(-pi, w.y, xp.x));
+    xp.y = fma(pr, w.y, fma(pi, w.x, xp.y));
+    xm.x = fma(qr, w.x, fma(qi, w.y, xm.x));
+    xm.y = fma(qi, w.x, fma(-qr, w.y, xm.y));
+    m += k;
+    if (m >= N) m -= N;
+  }
+}
+
 }  // namespace gx

@@ -1352,7 +1352,8 @@ __global__ __launch_bounds__(BLK) void k_colpass(gx_frames d, int64_t f0) {
 // h[t] = conj(c[k_lo + t]) wrapped (host, FP64, already divided by M); the inverse is
 // conj(FFT(conj(.))).  Output j of the inverse transform is X[k_lo + j].
 // ------------------------------------------------------------------------------------
-// per-frame background spectrum on the kept columns by a direct FP64 DFT
+// per-frame background spectrum on the kept columns by a direct FP64 DFT (dft_band_pair:
+// 892 frames at N = 1048, 275 -> 42 us against a twiddle gathered for every product)
 __global__ __launch_bounds__(BLK) void k_frames_spectra_dft(gx_frames d, int64_t f0) {
   GX_RESOLVE_AVG(d);
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -1385,23 +1386,25 @@ __global__ __launch_bounds__(BLK) void k_frames_spectra_dft(gx_frames d, int64_t
     }
     u[y] = make_double2(ure, uim);
   }
+  for (int y = N + threadIdx.x; y < dft_pad(N); y += BLK) u[y] = make_double2(0.0, 0.0);
   __syncthreads();
   const double2 *tw = reinterpret_cast<const double2 *>(d.twiddle64);
-  for (int w = threadIdx.x; w < wf; w += BLK) {
-    const int k = (jlo + w + N - N / 2) % N;  // unshifted frequency of column jlo + w
-    double re = 0.0, im = 0.0;
-    int m = 0;
-    for (int y = 0; y < N; ++y) {
-      const double2 t = tw[m], x = u[y];
-      re = fma(x.x, t.x, fma(-x.y, t.y, re));
-      im = fma(x.x, t.y, fma(x.y, t.x, im));
-      m += k;
-      if (m >= N) m -= N;
-    }
+  // |k| up to the band's larger end; column w holds the signed frequency klo + w
+  const int klo = jlo - N / 2, khi = jhi - N / 2;
+  auto put = [&](int k, double2 x) {
+    if (k < klo || k > khi) return;
+    const int64_t o = (int64_t)fb * d.W + (k - klo);
     if (d.fft_f64)
-      reinterpret_cast<double2 *>(d.col_spec)[(int64_t)fb * d.W + w] = make_double2(re, im);
+      reinterpret_cast<double2 *>(d.col_spec)[o] = x;
     else
-      reinterpret_cast<float2 *>(d.col_spec)[(int64_t)fb * d.W + w] = make_float2((float)re, (float)im);
+      reinterpret_cast<float2 *>(d.col_spec)[o] = make_float2((float)x.x, (float)x.y);
+  };
+  const int k0 = klo > 0 ? klo : khi < 0 ? -khi : 0, k1 = max(-klo, khi);
+  for (int k = k0 + threadIdx.x; k <= k1; k += BLK) {
+    double2 xp, xm;
+    dft_band_pair<true>(reinterpret_cast<const double *>(u), N, tw, k, xp, xm);
+    put(k, xp);
+    if (k > 0) put(-k, xm);
   }
 }
 
@@ -2264,7 +2267,7 @@ int gx_frames_columns(const gx_frames *d, int64_t f0, int64_t nf, gx_stream_t st
   rc = check_launch("gx_frames_columns");
   if (rc || !(d->fill_bkg || d->smooth)) return rc;
   if (d->bs_M) {
-    k_frames_spectra_dft<<<(unsigned)nf, BLK, (size_t)d->N * sizeof(double2), st>>>(*d, f0);
+    k_frames_spectra_dft<<<(unsigned)nf, BLK, (size_t)dft_pad((int)d->N) * sizeof(double2), st>>>(*d, f0);
     return check_launch("k_frames_spectra_dft");
   }
   switch (d->N) {
