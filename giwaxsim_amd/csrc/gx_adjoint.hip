@@ -1362,6 +1362,7 @@ void k_adj_rowpass_bsw(gx_frames d, gx_adjoint g, int64_t f0) {
   }
   // the band, staged in the wave's buffer
   const bool dense = d.fill_bkg || d.smooth;
+  const bool k0_apart = bs_k0_apart(d);
   const double avv_re = d.avg_re * d.max_voxels, avv_im = d.avg_im * d.max_voxels;
   const double mz = d.smooth ? d.col_sz[(int64_t)fb * N + v] : 1.0;
   const C *spec = reinterpret_cast<const C *>(d.col_spec) + (int64_t)fb * d.W;
@@ -1375,14 +1376,15 @@ void k_adj_rowpass_bsw(gx_frames d, gx_adjoint g, int64_t f0) {
     C o = C{(T)0, (T)0};
     if (atoms) o = cmul(x[q], chirp[k < 0 ? -k : k]);
     if (!inside) {
-      o = (k == 0) ? C{(T)(avv_re * (double)N), (T)(avv_im * (double)N)} : C{(T)0, (T)0};
+      o = (k == 0 && !k0_apart) ? C{(T)(avv_re * (double)N), (T)(avv_im * (double)N)} : C{(T)0, (T)0};
     } else if (dense) {
       const C u = spec[w];
       double ore = mz * ((double)o.x + (double)u.x);
       double oim = mz * ((double)o.y + (double)u.y);
-      if (d.smooth && k == 0) {
-        ore = ore + avv_re * (double)N;
-        oim = oim + avv_im * (double)N;
+      if (k == 0) {
+        const double m = (d.smooth ? 1.0 : 0.0) - (k0_apart ? 1.0 : 0.0);
+        ore = ore + m * (avv_re * (double)N);
+        oim = oim + m * (avv_im * (double)N);
       }
       o = C{(T)ore, (T)oim};
     }
@@ -1431,16 +1433,21 @@ __global__ __launch_bounds__(BLK) void k_adj_colpass_bsw(gx_frames d, gx_adjoint
   const double *sz_row = d.col_sz + (int64_t)fb * N;
   const C *chirp = reinterpret_cast<const C *>(d.bs_chirp);
   const C *tw = reinterpret_cast<const C *>(d.bs_twiddle_c);
-  C a0 = C{(T)0, (T)0};
-  if (k0 && dense)
-    a0 = C{(T)(d.avg_re * d.max_voxels * (double)N), (T)(d.avg_im * d.max_voxels * (double)N)};
+  const bool k0_apart = bs_k0_apart(d);
+  double2 A = make_double2(0.0, 0.0);
+  if (k0 && (d.fill_bkg || d.smooth))
+    A = make_double2(d.avg_re * d.max_voxels * (double)N, d.avg_im * d.max_voxels * (double)N);
+  const C a0 = C{(T)A.x, (T)A.y};
   const bool head = (d.fill_bkg || !d.smooth) && d.Z <= GX_WAVE * CHW_NZ;  // as k_colpass_bsw
   const int Lc = (int)min((int64_t)N, d.bs_Mc - d.bs_ck + 1);
   C v[CHW_P];
   auto load = [&](int q) {
     const int z = lane + GX_WAVE * q;
     v[q] = C{(T)0, (T)0};
-    if (z < Lc) v[q] = cmul(csub(col_input(d, (const C *)col, z, k0, u, sz_row), a0), chirp[z]);
+    if (z < Lc) {
+      const C e = col_input(d, (const C *)col, z, k0, u, sz_row);
+      v[q] = cmul(k0_apart && z < d.Z ? e : csub(e, a0), chirp[z]);
+    }
   };
   if (head) {
 #pragma unroll
@@ -1474,7 +1481,7 @@ __global__ __launch_bounds__(BLK) void k_adj_colpass_bsw(gx_frames d, gx_adjoint
           const double gI = 2.0 * g.g_bins[cbase + bz];
           C F = cmul(v[q], ck);
           if (k0 && k == 0)
-            F = C{(T)((double)F.x + (double)a0.x * (double)N), (T)((double)F.y + (double)a0.y * (double)N)};
+            F = C{(T)((double)F.x + A.x * (double)N), (T)((double)F.y + A.y * (double)N)};
           const double gr = gI * (double)F.x, gi = gI * (double)F.y;
           if (dense) {
             const double2 zh = zhat[kk];
