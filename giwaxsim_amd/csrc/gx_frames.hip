@@ -1000,7 +1000,10 @@ __global__ __launch_bounds__(BLK) void k_rowpass_blk(gx_frames d, int64_t f0, in
 // Rows per wave: more rows amortise the per-frame prologue (the smoothed y mask in
 // registers), but at N = 2048 a loop over rows keeps more than 256 registers live
 // (spills), while one row per wave is straight-line code (measured on the 1.3M-atom
-// slab: 0.61 ms per 119-frame launch with one row per wave, 1.08 ms with two).
+// slab: 0.61 ms per 119-frame launch with one row per wave, 1.08 ms with two).  There the waves
+// of a block take the same row of neighbouring frames, so its atoms (78 KB) reach the CU's L1
+// once for the four: 0.61 -> 0.56 ms.  With 8 waves per CU (18 KB of LDS each) the rest is
+// waiting: vector instructions issue 44% of the time.
 template <int N> struct RowRm {
   static constexpr int RPWV = (N <= 1024) ? 8 : 1;
   static constexpr int RB = (BLK / GX_WAVE) * RPWV;        // rows per block
@@ -1016,29 +1019,33 @@ void k_rowpass_rm(gx_frames d, int64_t f0, int64_t nf) {
   constexpr int RB = (BLK / GX_WAVE) * RPWV;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int lane = threadIdx.x & (GX_WAVE - 1);
-  const int wave = threadIdx.x / GX_WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / GX_WAVE);
   C *wbuf = reinterpret_cast<C *>(smem_raw) + wave * BUF;
   int32_t *acc_re = reinterpret_cast<int32_t *>(wbuf);
   int32_t *acc_im = acc_re + N;
 
   // tile order: frame major, or XCD-aware with the frames of a row block together (bit 2)
-  const int64_t nzb = gridDim.x / nf;
+  // (frame, row block); one row per wave: (frames of the block's waves, row)
+  constexpr int FW = RPWV == 1 ? BLK / GX_WAVE : 1;
+  const int64_t nfg = (nf + FW - 1) / FW, nzb = gridDim.x / nfg;
   int fb, zb;
   if (d.row_variant & 4) {
     const int64_t tile = xcd_tile(blockIdx.x, gridDim.x);
-    fb = (int)(tile % nf);
-    zb = (int)(tile / nf);
+    fb = (int)(tile % nfg);
+    zb = (int)(tile / nfg);
   } else {
     fb = (int)(blockIdx.x / nzb);
     zb = (int)(blockIdx.x % nzb);
   }
+  if (FW > 1) fb = fb * FW + wave;
+  if (fb >= nf) return;  // wave-uniform, as every return: the kernel has no block barrier
   const int64_t f = f0 + fb;
   const double *fp = d.fparams + f * GX_FP_STRIDE;
   const int jlo = (int)fp[GX_FP_JLO], jhi = (int)fp[GX_FP_JHI];
   const int wf = jhi - jlo + 1;
-  if (wf <= 0) return;  // block-uniform
+  if (wf <= 0) return;
   if (wf > d.W) {       // planner guarantees wf <= W; never write past a row
-    if (threadIdx.x == 0 && zb == 0) atomicAdd(&d.status[1], 1);
+    if (lane == 0 && zb == 0 && (FW > 1 || wave == 0)) atomicAdd(&d.status[1], 1);
     return;
   }
   const double s = fp[GX_FP_SIN], c = fp[GX_FP_COS];
@@ -1059,7 +1066,7 @@ void k_rowpass_rm(gx_frames d, int64_t f0, int64_t nf) {
     for (int q = 0; q < R0; ++q)
       my[t * R0 + q] = d.smooth ? (T)d.col_sy[(int64_t)fb * N + lane + GX_WAVE * t + q * (N / R0)] : (T)1;
 
-  const int zw = zb * RB + wave * RPWV;
+  const int zw = FW > 1 ? zb : zb * RB + wave * RPWV;
   for (int rr = 0; rr < RPWV; ++rr) {
     const int z = zw + rr;
     if (z >= d.Z) break;
@@ -2014,7 +2021,8 @@ int launch_rowpass_rm_x(const gx_frames *d, int64_t f0, int64_t nf, hipStream_t 
                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     attr_set = true;
   }
-  const unsigned nblk = (unsigned)(((d->Z + RB - 1) / RB) * nf);
+  const unsigned nblk = RPWV == 1 ? (unsigned)(d->Z * ((nf + BLK / GX_WAVE - 1) / (BLK / GX_WAVE)))
+                                  : (unsigned)(((d->Z + RB - 1) / RB) * nf);
   k_rowpass_rm<N, C, RPWV, WPE, PL><<<nblk, BLK, lds, st>>>(*d, f0, nf);
   return check_launch("k_rowpass_rm");
 }
