@@ -1221,8 +1221,8 @@ __global__ __launch_bounds__(GX_BLK_FFT) void k_adj_rowgrad_bs(gx_frames d, gx_a
 //
 // Against the block-wide forms (four points per thread, twenty block barriers a transform), one
 // evaluation of the fit geometry (N = 1048, 139,000 four-row blocks, 200,000 columns, FP32):
-// row pass 4.21 -> 2.17 ms, column adjoint 3.04 -> 1.76 ms, row gradient 9.22 -> 3.87 ms.  The
-// row and column passes issue vector instructions 65-75% of the time; the row gradient 60%, its
+// row pass 4.21 -> 1.82 ms, column adjoint 3.04 -> 1.74 ms, row gradient 9.22 -> 3.85 ms.  The
+// row and column passes issue vector instructions 65-85% of the time; the row gradient 60%, its
 // gather's LDS reads most of the rest.
 // ------------------------------------------------------------------------------------
 constexpr int CHW_RB = NWAVE;  // rows per block: one per wave
@@ -1242,7 +1242,7 @@ void k_adj_rowpass_bsw(gx_frames d, gx_adjoint g, int64_t f0) {
   C *bufs = reinterpret_cast<C *>(smem_raw);  // [RB][CHW_BUF]
   AU *accs = reinterpret_cast<AU *>(smem_raw);
   double *ftab = reinterpret_cast<double *>(bufs + RB * CHW_BUF);  // [n_elem][2]
-  C *cm = reinterpret_cast<C *>(ftab + 2 * g.n_elem);              // [1024] chirp times node mask (FP32)
+  C *cm = reinterpret_cast<C *>(ftab + 2 * g.n_elem);              // [chw_mask_len] chirp times node mask (FP32)
   __shared__ double rsc[RB];
   const int lane = threadIdx.x & (GX_WAVE - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / GX_WAVE);
@@ -1264,6 +1264,7 @@ void k_adj_rowpass_bsw(gx_frames d, gx_adjoint g, int64_t f0) {
   const int ya = d.fill_bkg ? (ylo == INT_MAX ? N : ylo + 1) : 0;
   const int yb = d.fill_bkg ? (yhi == INT_MIN ? 0 : yhi) : N;
   const bool head = bnd[1] + 1 < GX_WAVE * CHW_NZ;  // the frame's deposits end below (block-uniform)
+  const int L = chw_mask_len(d);  // beyond, the accumulators are zero
   auto chirp_mask = [&](int n) {
     C x = C{(T)0, (T)0};
     if (n < N && n >= ya && n < yb) {
@@ -1280,7 +1281,7 @@ void k_adj_rowpass_bsw(gx_frames d, gx_adjoint g, int64_t f0) {
 #pragma unroll
     for (int i = 0; i < CHW_M / BLK; ++i) {
       const int n = threadIdx.x + BLK * i;
-      if (!(head && n >= GX_WAVE * CHW_NZ)) cm[n] = chirp_mask(n);
+      if (n < L && !(head && n >= GX_WAVE * CHW_NZ)) cm[n] = chirp_mask(n);
     }
   }
   if (threadIdx.x < RB) rsc[threadIdx.x] = ldexp(1.0, g.row_exp[min(z0 + (int)threadIdx.x, N - 1)]);
@@ -1345,7 +1346,7 @@ void k_adj_rowpass_bsw(gx_frames d, gx_adjoint g, int64_t f0) {
     auto load = [&](int q) {
       const int n = lane + GX_WAVE * q;
       x[q] = cmul(C{(T)((double)(AT)ar[n] * inv), (T)((double)(AT)ar[CHW_M + n] * inv)},
-                  sizeof(C) == 8 ? cm[n] : chirp_mask(n));
+                  sizeof(C) == 8 ? cm[min(n, L - 1)] : chirp_mask(n));
     };
     if (head) {
 #pragma unroll
@@ -1939,7 +1940,7 @@ int launch_adj_bsw(Op op, const gx_frames *d, const gx_adjoint *g, int64_t f0, i
   }
   const size_t lds = (size_t)NWAVE * CHW_BUF * sizeof(C) + (size_t)g->n_elem * 16;
   if (op == OP_ROWPASS) {
-    const size_t cm = sizeof(C) == 8 ? CHW_M * sizeof(C) : 0;
+    const size_t cm = sizeof(C) == 8 ? chw_mask_len(*d) * sizeof(C) : 0;
     k_adj_rowpass_bsw<C, G><<<dim3((unsigned)(d->Z / CHW_RB), (unsigned)nf), BLK, lds + cm, st>>>(*d, *g, f0);
     return check_launch("k_adj_rowpass_bsw");
   }

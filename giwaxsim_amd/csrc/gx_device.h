@@ -826,6 +826,14 @@ __device__ __forceinline__ double2 chirpz_fill_tail(const gx_frames &d, int kk, 
   return make_double2(tre * qre - tim * qim, tre * qim + tim * qre);
 }
 
+// Rows of the masked chirp that the row passes of length 1024 share in LDS: those that can hold
+// a deposit (y <= bs_M - bs_rk, checked per frame).  At 290 frequencies 736 rows, with which
+// four blocks fit a CU's LDS instead of three.
+__host__ __device__ __forceinline__ int chw_mask_len(const gx_frames &d) {
+  const int n = ((int)(d.bs_M - d.bs_rk) + 1 + 15) / 16 * 16;
+  return n < 16 ? 16 : n < CHW_M ? n : CHW_M;
+}
+
 // Whether the row pass leaves the k = 0 column's constant A N out of the intermediate, for the
 // column passes to add as the one value A N^2 that it transforms to: stored with it, the column's
 // FP32 values would be rounded to a multiple of its last bit.  Both passes of length 1024.

@@ -1565,9 +1565,10 @@ void k_rowpass_bs(gx_frames d, int64_t f0) {
 // The block-wide form spent a row in 20 block barriers at four points per thread.  Here a row
 // stays in one wave's registers and private LDS, its four rows share the masked chirp in LDS
 // (FP32), and the band is staged in the exchange buffers, so four blocks share a CU: 556,000
-// rows at N = 1048 (fit geometry, FP32) 4.22 -> 1.89 ms, about 1,700 vector instructions a row
-// at 90% of their issue rate.  More rows per wave one after another were slower (their table
-// indices held 50 more registers: two rows 4.5 ms per evaluation against 3.2).
+// rows at N = 1048 (fit geometry, FP32) 4.22 -> 1.59 ms, about 1,700 vector instructions a row
+// (1.85 ms with three blocks a CU, the chirp table at its full 8 KB).  More rows per wave one
+// after another were slower (their table indices held 50 more registers: two rows 4.5 ms per
+// evaluation against 3.2).
 template <typename C, int G>
 __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(sizeof(C) == 8 ? 4 : 2)))
 void k_rowpass_bsw(gx_frames d, int64_t f0) {
@@ -1578,7 +1579,7 @@ void k_rowpass_bsw(gx_frames d, int64_t f0) {
   const int lane = threadIdx.x & (GX_WAVE - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / GX_WAVE);
   C *bufs = reinterpret_cast<C *>(smem_raw), *fbuf = bufs + wave * CHW_BUF;
-  C *cm = bufs + RB * CHW_BUF;  // [1024] chirp times the smoothed y mask
+  C *cm = bufs + RB * CHW_BUF;  // [chw_mask_len] chirp times the smoothed y mask
   int32_t *acc_re = reinterpret_cast<int32_t *>(fbuf), *acc_im = acc_re + CHW_M;
   const int N = (int)d.N;
   const int fb = blockIdx.y;
@@ -1604,6 +1605,7 @@ void k_rowpass_bsw(gx_frames d, int64_t f0) {
       reinterpret_cast<int4 *>(acc_re)[lane + GX_WAVE * i] = make_int4(0, 0, 0, 0);
   }
   const bool head = bnd[1] < GX_WAVE * CHW_NZ;  // the frame's atoms end below (block-uniform)
+  const int L = chw_mask_len(d);  // beyond, the accumulators are zero
   auto chirp_mask = [&](int n) {
     C x = C{(T)0, (T)0};
     if (n < N) {
@@ -1620,7 +1622,7 @@ void k_rowpass_bsw(gx_frames d, int64_t f0) {
 #pragma unroll
     for (int i = 0; i < CHW_M / BLK; ++i) {
       const int n = threadIdx.x + BLK * i;
-      if (!(head && n >= GX_WAVE * CHW_NZ)) cm[n] = chirp_mask(n);
+      if (n < L && !(head && n >= GX_WAVE * CHW_NZ)) cm[n] = chirp_mask(n);
     }
     __syncthreads();
   } else {
@@ -1661,7 +1663,7 @@ void k_rowpass_bsw(gx_frames d, int64_t f0) {
     const T inv = (T)ldexp(1.0, -d.row_exp[z]);
     auto load = [&](int q) {
       const int n = lane + GX_WAVE * q;
-      v[q] = cmul(C{(T)acc_re[n] * inv, (T)acc_im[n] * inv}, sizeof(C) == 8 ? cm[n] : chirp_mask(n));
+      v[q] = cmul(C{(T)acc_re[n] * inv, (T)acc_im[n] * inv}, sizeof(C) == 8 ? cm[min(n, L - 1)] : chirp_mask(n));
     };
     if (head) {
 #pragma unroll
@@ -1890,7 +1892,7 @@ int launch_rowpass_bs_t(const gx_frames *d, int64_t f0, int64_t nf, hipStream_t 
 template <typename C, int G>
 int launch_rowpass_bsw(const gx_frames *d, int64_t f0, int64_t nf, hipStream_t st) {
   constexpr int RB = BLK / GX_WAVE;
-  const size_t lds = ((size_t)RB * CHW_BUF + (sizeof(C) == 8 ? CHW_M : 0)) * sizeof(C);  // staged rows: W <= bs_rk <= 1024
+  const size_t lds = ((size_t)RB * CHW_BUF + (sizeof(C) == 8 ? chw_mask_len(*d) : 0)) * sizeof(C);  // staged rows: W <= bs_rk <= 1024
   static bool attr_set = false;
   if (!attr_set) {
     GX_HIP(hipFuncSetAttribute((const void *)k_rowpass_bsw<C, G>, hipFuncAttributeMaxDynamicSharedMemorySize,
