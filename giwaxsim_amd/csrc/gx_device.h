@@ -524,7 +524,7 @@ __device__ __forceinline__ void fft_wave_kept(C (&v)[N / GX_WAVE], C *lds, const
 }
 
 // ------------------------------------------------------------------------------------
-// Block-level Stockham transforms of length M over GX_BLK_FFT = 256 threads
+// Block-level Stockham transforms of length M = 2048 or 4096 over GX_BLK_FFT = 256 threads
 // (P = M / 256 points per thread), used by the chirp-z (Bluestein) path for
 // grid edges that are not powers of two.  The plans have equal first and last
 // radix, so a transform's output registers are already laid out as the next
@@ -533,7 +533,6 @@ __device__ __forceinline__ void fft_wave_kept(C (&v)[N / GX_WAVE], C *lds, const
 // ------------------------------------------------------------------------------------
 #define GX_BLK_FFT 256
 template <int M> struct BlkPlan;
-template <> struct BlkPlan<1024> { static constexpr int R = 4; static constexpr int NST = 5; };   // 4^5
 template <> struct BlkPlan<2048> { static constexpr int R = 8; static constexpr int NST = 4; };   // 8 4 8 8
 template <> struct BlkPlan<4096> { static constexpr int R = 16; static constexpr int NST = 3; };  // 16^3
 
@@ -541,21 +540,7 @@ template <int M, typename C>
 __device__ __forceinline__ void fft_block(C (&v)[M / GX_BLK_FFT], C* lds, const C* __restrict__ tw, int tid) {
   constexpr int P = M / GX_BLK_FFT;
   constexpr int L = GX_BLK_FFT;
-  if constexpr (M == 1024) {
-    fft_butterflies<M, 4, 1, P, C, L>(v, tw, tid);
-    fft_store<M, 4, 1, P, C, L>(v, lds, tid); __syncthreads();
-    fft_load<M, 4, P, C, L>(v, lds, tid); __syncthreads();
-    fft_butterflies<M, 4, 4, P, C, L>(v, tw, tid);
-    fft_store<M, 4, 4, P, C, L>(v, lds, tid); __syncthreads();
-    fft_load<M, 4, P, C, L>(v, lds, tid); __syncthreads();
-    fft_butterflies<M, 4, 16, P, C, L>(v, tw, tid);
-    fft_store<M, 4, 16, P, C, L>(v, lds, tid); __syncthreads();
-    fft_load<M, 4, P, C, L>(v, lds, tid); __syncthreads();
-    fft_butterflies<M, 4, 64, P, C, L>(v, tw, tid);
-    fft_store<M, 4, 64, P, C, L>(v, lds, tid); __syncthreads();
-    fft_load<M, 4, P, C, L>(v, lds, tid); __syncthreads();
-    fft_butterflies<M, 4, 256, P, C, L>(v, tw, tid);
-  } else if constexpr (M == 2048) {
+  if constexpr (M == 2048) {
     fft_butterflies<M, 8, 1, P, C, L>(v, tw, tid);
     fft_store<M, 8, 1, P, C, L>(v, lds, tid); __syncthreads();
     fft_load<M, 4, P, C, L>(v, lds, tid); __syncthreads();
