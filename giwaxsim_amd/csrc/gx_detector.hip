@@ -1377,9 +1377,16 @@ int gx_detector_accumulate(const gx_detector *d, gx_stream_t stream) {
   return check_launch("gx_detector_accumulate");
 }
 
-// 24-bit products of grid edges, 32-bit byte offsets and orientation indices
+// The linear maps need 24-bit products of grid edges, 32-bit byte offsets and orientation indices.
+// Below 40 orientations and 2^25 samples the launch that forms the maps costs more than they
+// save: 150^2 px x 5 0.094 against 0.104 ms, 250^2 x 20 0.099 against 0.102; above the line
+// 60^2 x 40 0.114 against 0.112, 700^2 x 40 0.140 against 0.119, 1400^2 x 30 0.228 against 0.169.
+// Where k_detector_coop runs without them, from 160 orientations: 250^2 x 90 0.119 against 0.128,
+// 150^2 x 120 0.123 against 0.129, 150^2 x 200 0.145 against 0.134, 250^2 x 181 0.141 against 0.130.
 static bool det_linear(const gx_detector *d) {
   const int64_t side = std::max(std::max(d->cx, d->cy), d->cz);
+  if (d->n_orient < 40 && d->n_pix * d->n_pix * d->n_orient < (1ll << 25)) return false;
+  if (d->n_orient >= COOP_MIN_ORIENT && d->n_orient < 160 && d->n_pix * d->n_pix <= COOP_MAX_PIX) return false;
   return d->n_orient >= 1 && d->n_orient <= (1 << 24) && side < (1 << 12) &&
          d->cy * d->cx * d->cz * (d->iq_f64 ? 8 : 4) < (1ll << 32);
 }

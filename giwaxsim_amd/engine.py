@@ -1055,10 +1055,11 @@ def detector_plan(num_pixels, max_q, angle_init_vals, angle_init_axs, psis, psi_
 
 
 def detector_work(desc):
-    """The work buffer of gx_detector_accumulate_ws for a detector descriptor."""
+    """The work buffer of gx_detector_accumulate_ws for a detector descriptor (None where it
+    takes none)."""
     n = ctypes.c_int64(0)
     call("gx_detector_work_size", ctypes.byref(desc), ctypes.byref(n))
-    return _empty(n.value, torch.float64)
+    return _empty(n.value, torch.float64) if n.value else None
 
 
 def run_detector(iq_dev, qx, qy, qz, plan: DetectorPlan, mirror, floor_scale=True):

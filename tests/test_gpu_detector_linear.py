@@ -113,3 +113,15 @@ def test_exact_chain_cases(kind):
         more = dict(orient_R=Q)
     a, b = _both(plan, iq, q0, dq, **more)
     assert np.array_equal(a, b, equal_nan=True)
+
+
+@pytest.mark.parametrize("n_pix,n_orient", [(15, 39), (15, 40), (33, 63), (33, 64), (33, 159), (33, 160), (1, 160),
+                                            (49, 163), (64, 257), (362, 64), (363, 64)])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_both_sides_of_the_size_rule(n_pix, n_orient, dtype):
+    """Orientation counts and image sizes at the lines where the linear maps take over from the
+    plain kernels and from their cooperative form."""
+    print(f"[gpu-detector-linear] rule: {n_pix} px, {n_orient} orientations, {dtype}", flush=True)
+    a, b = _both(_plan(n_pix, np.linspace(0.0, 173.0, n_orient), ONE, ONE), _grid((61, 47, 83), dtype), (-1.1, -1.5, -2.0),
+                 0.04)
+    assert np.array_equal(a, b, equal_nan=True)
