@@ -116,7 +116,8 @@ def test_exact_chain_cases(kind):
 
 
 @pytest.mark.parametrize("n_pix,n_orient", [(15, 39), (15, 40), (33, 63), (33, 64), (33, 159), (33, 160), (1, 160),
-                                            (49, 163), (64, 257), (362, 64), (363, 64)])
+                                            (49, 163), (64, 257), (362, 64), (363, 64),
+                                            (14, 40), (34, 160), (50, 163), (2, 200), (599, 41), (601, 41), (601, 64)])
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 def test_both_sides_of_the_size_rule(n_pix, n_orient, dtype):
     """Orientation counts and image sizes at the lines where the linear maps take over from the
