@@ -1383,14 +1383,17 @@ int gx_detector_accumulate(const gx_detector *d, gx_stream_t stream) {
 // 60^2 x 40 0.114 against 0.112, 700^2 x 40 0.140 against 0.119, 1400^2 x 30 0.228 against 0.169.
 // Where k_detector_coop runs without them, from 160 orientations: 250^2 x 90 0.119 against 0.128,
 // 150^2 x 120 0.123 against 0.129, 150^2 x 200 0.145 against 0.134, 250^2 x 181 0.141 against 0.130.
-// An odd image has a middle row and column at q = 0, whose samples lie on voxel planes and take the
-// exact path at every orientation: below 600 px or 2^25 samples their waves finish last (483^2 px x
-// 52 0.135 against 0.169 ms, 197^2 x 246 0.154 against 0.185, 727^2 x 40 0.162 against 0.171;
-// 877^2 x 45 0.184 against 0.179, 653^2 x 1,430 2.14 against 0.94).
+// An odd image has pixels at q = 0 (its centre, in some geometries the middle row or column), which
+// lie on voxel planes at every orientation: they take the exact chain and their waves finish last.
+// Kernel times, plain against maps, from 61 to 901 px: at 251 px two angles 0.219 against 0.272 ms
+// (x 721), 4.60 against 5.70 (x 16,000), one angle 4.37 against 3.67; at 299 px two angles 0.318
+// against 0.249 (x 721), 6.88 against 5.01 (x 16,000), one angle 6.24 against 4.02; at 499 px 3.25
+// against 1.54 (two angles x 3,000).  Below 2^25 samples either may win: 299^2 x 200 0.098 against
+// 0.107, 401^2 x 200 0.185 against 0.105, 701^2 x 60 0.085 against 0.097.
 static bool det_linear(const gx_detector *d) {
   const int64_t side = std::max(std::max(d->cx, d->cy), d->cz);
   const bool large = d->n_pix * d->n_pix * d->n_orient >= (1ll << 25), odd = d->n_pix & 1;
-  if (odd ? !large || d->n_pix < 600 : !large && d->n_orient < 40) return false;
+  if (odd ? !large || d->n_pix < 290 : !large && d->n_orient < 40) return false;
   if (d->n_orient >= COOP_MIN_ORIENT && d->n_orient < 160 && d->n_pix * d->n_pix <= COOP_MAX_PIX) return false;
   return d->n_orient >= 1 && d->n_orient <= (1 << 24) && side < (1 << 12) &&
          d->cy * d->cx * d->cz * (d->iq_f64 ? 8 : 4) < (1ll << 32);

@@ -98,6 +98,17 @@ def test_planes_on_boundaries(init, angles):
     assert np.array_equal(a, b)
 
 
+def test_odd_image_on_boundaries():
+    """An odd image on the map side: its own middle row and column lie at q = 0."""
+    print("[gpu-detector-route] 401 px, 9 psi x 24 phi, stand", flush=True)
+    q = np.linspace(-2.0, 2.0, 101)
+    plan = _plan(401, np.linspace(0.0, 90.0, 9), np.linspace(0.0, 179.0, 24), (0.0,), 'stand', 1.96)
+    assert 0.0 in plan.h and 0.0 in plan.v
+    a, b, mapped = _images(plan, _grid((101, 101, 101), torch.float64), (q[0],) * 3, float(np.diff(q)[0]))
+    assert mapped
+    assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("size", [COOP, DIRECT])
 @pytest.mark.parametrize("kind", ['lattice', 'outside', 'far', 'inf', 'nan_axis', 'nan_grid', 'big_matrix', 'nan_matrix',
                                   'offset'])
