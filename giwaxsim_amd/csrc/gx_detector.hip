@@ -546,7 +546,7 @@ struct DetLane {
     }
     const char *__restrict__ iq = reinterpret_cast<const char *>(d.iq);
 #pragma unroll
-    for (int j = 0; j < U * P; ++j) out[j] = *reinterpret_cast<const T *>(iq + (uint32_t)(vox[j] * (int)sizeof(T)));
+    for (int j = 0; j < U * P; ++j) out[j] = *reinterpret_cast<const T *>(iq + (uint32_t)vox[j] * (uint32_t)sizeof(T));
   }
 };
 

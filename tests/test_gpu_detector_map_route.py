@@ -149,3 +149,17 @@ def test_exact_chain(kind, size):
     a, b, mapped = _images(plan, iq, q0, dq, **more)
     assert mapped
     assert np.array_equal(a, b, equal_nan=True)
+
+
+def test_grid_beyond_two_gib():
+    """Byte offsets of the maps' gathers beyond 2^31: an FP64 grid of 647^3, zero below them."""
+    print("[gpu-detector-route] 647^3 FP64 grid, 300 px, 181 orientations", flush=True)
+    iq = _grid((647, 647, 647), torch.float64)
+    low = 642  # first index whose whole slab lies beyond
+    assert low * 647 * 647 * 8 >= 2 ** 31
+    iq[:low] = 0.0
+    q = np.linspace(-2.0, 2.0, 647)
+    a, b, mapped = _images(_plan(300, np.linspace(0.0, 180.0, 181), max_q=2.1), iq, (q[0],) * 3, float(np.diff(q)[0]))
+    assert mapped
+    assert np.count_nonzero(a) > 1000
+    assert np.array_equal(a, b)
