@@ -123,8 +123,11 @@ template <int R, typename C> struct Dft;
 
 template <typename T> struct DftConst {
   static constexpr T c2 = (T)0.70710678118654752440, t = (T)0.41421356237309504880;
-  // cos(pi / 8); in FP32 the neighbour above, whose error offsets that of c2: the mean gain of a
-  // 1024-point transform is 1 - 4e-9, with the nearest value 1 - 3.5e-8
+  // cos(pi / 8); in FP32 the neighbour above, whose error offsets that of c2.  The constants' rounding
+  // acts on every frame alike: over the matrix of a 1024-point transform the mean gain is 1 - 4e-9 and
+  // the rms error 3.7e-8 (16.4.16), with the nearest value 1 - 3.7e-8 and 5.0e-8; the other plans with
+  // a radix of 16 likewise.  dL/df of the differentiable path at N = 1024 and 2048, FP32 against FP64:
+  // under 1e-7, with the nearest value 2e-6 to 5e-6.
   static constexpr T c1 = sizeof(T) == 4 ? (T)0.923879563808441162109375 : (T)0.92387953251128675613;
 };
 // a = e + c z, b = e - c z
