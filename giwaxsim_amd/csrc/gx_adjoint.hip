@@ -1446,8 +1446,8 @@ __global__ __launch_bounds__(BLK) void k_adj_colpass_bsw(gx_frames d, gx_adjoint
     const int z = lane + GX_WAVE * q;
     v[q] = C{(T)0, (T)0};
     if (z < Lc) {
-      const C e = col_input(d, (const C *)col, z, k0, u, sz_row);
-      v[q] = cmul(k0_apart && z < d.Z ? e : csub(e, a0), chirp[z]);
+      const C e = col_input(d, (const C *)col, z, false, u, sz_row);  // without A N from row Z on
+      v[q] = cmul(k0_apart || z >= d.Z ? e : csub(e, a0), chirp[z]);
     }
   };
   if (head) {

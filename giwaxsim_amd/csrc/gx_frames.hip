@@ -1733,9 +1733,10 @@ void k_rowpass_bsw(gx_frames d, int64_t f0) {
 
 // The column pass for bands of length 1024: a wave per kept column, no block barriers (fit
 // geometry, 200,000 columns: 1.10 -> 0.81 ms; the atomics take 0.2 ms of it).  The k = 0
-// column's background A N is subtracted on every row and its transform, A N^2 at k_z = 0, added:
-// it needs no tail beyond the band and does not cancel in FP32 (its weak voxels' error 2e-5 ->
-// under 1e-5 of themselves).
+// column's background A N is left out of every row (subtracted from those of the row pass where
+// that one's length is not 1024) and its transform, A N^2 at k_z = 0, added: it needs no tail
+// beyond the band, and FP32 rows hold no multiple of it (N = 700, central line of I(q): rms error
+// 1e-5 to 4e-5 -> 5e-7 to 3e-6 with fill, 5e-6 -> 3e-7 without, of themselves).
 template <typename C, int G>
 __global__ __launch_bounds__(BLK) void k_colpass_bsw(gx_frames d, int64_t f0) {
   GX_RESOLVE_AVG(d);
@@ -1776,8 +1777,8 @@ __global__ __launch_bounds__(BLK) void k_colpass_bsw(gx_frames d, int64_t f0) {
     const int z = lane + GX_WAVE * q;
     v[q] = C{(T)0, (T)0};
     if (z < Lc) {
-      const C e = col_input(d, col, z, k0, u, sz_row);
-      v[q] = cmul(k0_apart && z < d.Z ? e : csub(e, a0), chirp[z]);
+      const C e = col_input(d, col, z, false, u, sz_row);  // without A N from row Z on
+      v[q] = cmul(k0_apart || z >= d.Z ? e : csub(e, a0), chirp[z]);
     }
   };
   if (head) {
