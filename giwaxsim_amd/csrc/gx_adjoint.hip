@@ -1221,7 +1221,7 @@ __global__ __launch_bounds__(GX_BLK_FFT) void k_adj_rowgrad_bs(gx_frames d, gx_a
 //
 // Against the block-wide forms (four points per thread, twenty block barriers a transform), one
 // evaluation of the fit geometry (N = 1048, 139,000 four-row blocks, 200,000 columns, FP32):
-// row pass 4.21 -> 1.82 ms, column adjoint 3.04 -> 1.74 ms, row gradient 9.22 -> 3.85 ms.  The
+// row pass 4.21 -> 1.82 ms, column adjoint 3.04 -> 1.37 ms, row gradient 9.22 -> 3.85 ms.  The
 // row and column passes issue vector instructions 65-85% of the time; the row gradient 60%, its
 // gather's LDS reads most of the rest.
 // ------------------------------------------------------------------------------------
@@ -1263,7 +1263,7 @@ void k_adj_rowpass_bsw(gx_frames d, gx_adjoint g, int64_t f0) {
   const int ylo = bnd[0], yhi = bnd[1], zlo = bnd[2], zhi = bnd[3];
   const int ya = d.fill_bkg ? (ylo == INT_MAX ? N : ylo + 1) : 0;
   const int yb = d.fill_bkg ? (yhi == INT_MIN ? 0 : yhi) : N;
-  const bool head = bnd[1] + 1 < GX_WAVE * CHW_NZ;  // the frame's deposits end below (block-uniform)
+  const int used = bnd[1] == INT_MIN ? 0 : bnd[1] + 2;  // the frame's deposits end below (block-uniform)
   const int L = chw_mask_len(d);  // beyond, the accumulators are zero
   auto chirp_mask = [&](int n) {
     C x = C{(T)0, (T)0};
@@ -1281,7 +1281,7 @@ void k_adj_rowpass_bsw(gx_frames d, gx_adjoint g, int64_t f0) {
 #pragma unroll
     for (int i = 0; i < CHW_M / BLK; ++i) {
       const int n = threadIdx.x + BLK * i;
-      if (n < L && !(head && n >= GX_WAVE * CHW_NZ)) cm[n] = chirp_mask(n);
+      if (n < L && n < chw_read(used)) cm[n] = chirp_mask(n);
     }
   }
   if (threadIdx.x < RB) rsc[threadIdx.x] = ldexp(1.0, g.row_exp[min(z0 + (int)threadIdx.x, N - 1)]);
@@ -1348,15 +1348,7 @@ void k_adj_rowpass_bsw(gx_frames d, gx_adjoint g, int64_t f0) {
       x[q] = cmul(C{(T)((double)(AT)ar[n] * inv), (T)((double)(AT)ar[CHW_M + n] * inv)},
                   sizeof(C) == 8 ? cm[min(n, L - 1)] : chirp_mask(n));
     };
-    if (head) {
-#pragma unroll
-      for (int q = 0; q < CHW_NZ; ++q) load(q);
-      DftHead<16, CHW_NZ, C>::run(x);
-    } else {
-#pragma unroll
-      for (int q = 0; q < CHW_P; ++q) load(q);
-      DftHead<16, CHW_P, C>::run(x);
-    }
+    chw_first(x, used, load);
     wave_sync();
     chirpz_wave<C>(x, fbuf, reinterpret_cast<const C *>(d.bs_kernel), reinterpret_cast<const C *>(d.bs_twiddle), lane);
     wave_sync();
@@ -1438,26 +1430,26 @@ __global__ __launch_bounds__(BLK) void k_adj_colpass_bsw(gx_frames d, gx_adjoint
   double2 A = make_double2(0.0, 0.0);
   if (k0 && (d.fill_bkg || d.smooth))
     A = make_double2(d.avg_re * d.max_voxels * (double)N, d.avg_im * d.max_voxels * (double)N);
-  const C a0 = C{(T)A.x, (T)A.y};
-  const bool head = (d.fill_bkg || !d.smooth) && d.Z <= GX_WAVE * CHW_NZ;  // as k_colpass_bsw
-  const int Lc = (int)min((int64_t)N, d.bs_Mc - d.bs_ck + 1);
+  const C a0 = k0_apart ? C{(T)0, (T)0} : C{(T)A.x, (T)A.y};
+  const bool spread = !d.fill_bkg && d.smooth;  // background beyond the rows of the row pass
+  const int Lc = (int)min((int64_t)N, d.bs_Mc - d.bs_ck + 1), rows = min((int)d.Z, Lc);
   C v[CHW_P];
-  auto load = [&](int q) {
-    const int z = lane + GX_WAVE * q;
-    v[q] = C{(T)0, (T)0};
-    if (z < Lc) {
-      const C e = col_input(d, (const C *)col, z, false, u, sz_row);  // without A N from row Z on
-      v[q] = cmul(k0_apart || z >= d.Z ? e : csub(e, a0), chirp[z]);
-    }
-  };
-  if (head) {
-#pragma unroll
-    for (int q = 0; q < CHW_NZ; ++q) load(q);
-    DftHead<16, CHW_NZ, C>::run(v);
+  if (spread) {
+    chw_first(v, CHW_M, [&](int q) {
+      const int z = lane + GX_WAVE * q;
+      v[q] = C{(T)0, (T)0};
+      if (z < Lc) {
+        const C e = col_input(d, (const C *)col, z, false, u, sz_row);  // without A N from row Z on
+        v[q] = cmul(z >= rows ? e : csub(e, a0), chirp[z]);
+      }
+    });
   } else {
-#pragma unroll
-    for (int q = 0; q < CHW_P; ++q) load(q);
-    DftHead<16, CHW_P, C>::run(v);
+    // no branch between the loads: all of them are in flight at once
+    chw_first(v, rows, [&](int q) {
+      const int z = lane + GX_WAVE * q, zc = min(z, rows - 1);
+      const C e = csub(col[zc], a0);
+      v[q] = cmul(z < rows ? e : C{(T)0, (T)0}, chirp[zc]);
+    });
   }
   chirpz_wave<C>(v, lds[wave], reinterpret_cast<const C *>(d.bs_kernel_c), tw, lane);
   const int64_t cbase = (by * d.c_n + bx) * d.c_n;
@@ -1953,9 +1945,8 @@ int dispatch_bs_c(Op op, const gx_frames *d, const gx_adjoint *g, int64_t f0, in
   const int64_t M = (op == OP_COLPASS) ? d->bs_Mc : d->bs_M;
   switch (M) {
     case 1024:
-      return (op == OP_COLPASS ? d->bs_ck : d->bs_rk) <= GX_WAVE * CHW_G
-                 ? launch_adj_bsw<C, CHW_G>(op, d, g, f0, nf, st)
-                 : launch_adj_bsw<C, CHW_P>(op, d, g, f0, nf, st);
+      return chw_band(op == OP_COLPASS ? d->bs_ck : d->bs_rk,
+                      [&](auto G) { return launch_adj_bsw<C, G>(op, d, g, f0, nf, st); });
     case 2048: return launch_adj_bs_t<2048, C>(op, d, g, f0, nf, st);
     case 4096: return launch_adj_bs_t<4096, C>(op, d, g, f0, nf, st);
     default: return set_error(GX_ERR_UNSUPPORTED, "chirp-z transform length %lld", (long long)M);

@@ -10,6 +10,7 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 #include "../../include/giwaxsim_amd.h"
 
@@ -597,10 +598,34 @@ __device__ __forceinline__ void chirpz_block(C (&v)[M / GX_BLK_FFT], C *lds, con
 // ------------------------------------------------------------------------------------
 constexpr int CHW_M = 1024, CHW_P = CHW_M / GX_WAVE;
 constexpr int CHW_BUF = CHW_M + CHW_M / 16;  // complex values of a wave's exchange buffer
-// The first butterflies have a form for inputs of up to CHW_NZ groups of 64 points, and the
-// kernels are compiled for bands of up to CHW_G groups and for all 16: at the fit geometry 603
-// rows and 290 frequencies (10 and 5 groups).
-constexpr int CHW_NZ = 10, CHW_G = 5;
+// Inputs and bands count in groups of 64 values.  The first butterflies have a form without the
+// operations on zeros for every second number of groups, the kernels a form without the unused
+// outputs for every fourth (a band step of 1 or 2 measured the same; an input step of 4 against 2:
+// 2.57 against 2.53 ms a call at 603 rows, N = 1048, 0.317 against 0.305 at 225 rows, N = 700).
+constexpr int CHW_STEP = 2, CHW_BAND = 4;
+
+// the first butterflies of n inputs: load(r) fills v[r]
+template <int NZ = CHW_STEP, typename C, typename F>
+__device__ __forceinline__ void chw_first(C (&v)[CHW_P], int n, F load) {
+  if constexpr (NZ < CHW_P) {
+    if (n > GX_WAVE * NZ) return chw_first<NZ + CHW_STEP>(v, n, load);
+  }
+#pragma unroll
+  for (int r = 0; r < NZ; ++r) load(r);
+  DftHead<16, NZ, C>::run(v);
+}
+// values that chw_first reads for n inputs
+__device__ __forceinline__ int chw_read(int n) {
+  constexpr int S = GX_WAVE * CHW_STEP;
+  return min((max(n, 1) + S - 1) / S * S, CHW_M);
+}
+// f(integral constant) with the groups that hold a band of n values
+template <int G = CHW_BAND, typename F> auto chw_band(int64_t n, F f) {
+  if constexpr (G < CHW_P) {
+    if (n > GX_WAVE * G) return chw_band<G + CHW_BAND>(n, f);
+  }
+  return f(std::integral_constant<int, G>());
+}
 
 // The transform after its first butterflies (DftHead<16> on v[r] = x[lane + 64 r], which the
 // caller runs for as many inputs as may not be zero) -> v[r] = X[lane + 64 r]; the buffer is

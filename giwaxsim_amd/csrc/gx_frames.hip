@@ -1604,7 +1604,7 @@ void k_rowpass_bsw(gx_frames d, int64_t f0) {
     for (int i = 0; i < (2 * CHW_M) / (4 * GX_WAVE); ++i)
       reinterpret_cast<int4 *>(acc_re)[lane + GX_WAVE * i] = make_int4(0, 0, 0, 0);
   }
-  const bool head = bnd[1] < GX_WAVE * CHW_NZ;  // the frame's atoms end below (block-uniform)
+  const int used = bnd[1] == INT_MIN ? 0 : bnd[1] + 1;  // the frame's atoms end below (block-uniform)
   const int L = chw_mask_len(d);  // beyond, the accumulators are zero
   auto chirp_mask = [&](int n) {
     C x = C{(T)0, (T)0};
@@ -1622,7 +1622,7 @@ void k_rowpass_bsw(gx_frames d, int64_t f0) {
 #pragma unroll
     for (int i = 0; i < CHW_M / BLK; ++i) {
       const int n = threadIdx.x + BLK * i;
-      if (n < L && !(head && n >= GX_WAVE * CHW_NZ)) cm[n] = chirp_mask(n);
+      if (n < L && n < chw_read(used)) cm[n] = chirp_mask(n);
     }
     __syncthreads();
   } else {
@@ -1679,15 +1679,7 @@ void k_rowpass_bsw(gx_frames d, int64_t f0) {
       const int n = lane + GX_WAVE * q;
       v[q] = cmul(C{(T)acc_re[n] * inv, (T)acc_im[n] * inv}, sizeof(C) == 8 ? cm[min(n, L - 1)] : chirp_mask(n));
     };
-    if (head) {
-#pragma unroll
-      for (int q = 0; q < CHW_NZ; ++q) load(q);
-      DftHead<16, CHW_NZ, C>::run(v);
-    } else {
-#pragma unroll
-      for (int q = 0; q < CHW_P; ++q) load(q);
-      DftHead<16, CHW_P, C>::run(v);
-    }
+    chw_first(v, used, load);
     wave_sync();
     chirpz_wave<C>(v, fbuf, reinterpret_cast<const C *>(d.bs_kernel),
                        reinterpret_cast<const C *>(d.bs_twiddle), lane);
@@ -1732,7 +1724,8 @@ void k_rowpass_bsw(gx_frames d, int64_t f0) {
 }
 
 // The column pass for bands of length 1024: a wave per kept column, no block barriers (fit
-// geometry, 200,000 columns: 1.10 -> 0.81 ms; the atomics take 0.2 ms of it).  The k = 0
+// geometry, 200,000 columns: 1.10 -> 0.70 ms, 0.83 with a branch around each load; the atomics
+// take 0.2 ms of it).  The k = 0
 // column's background A N is left out of every row (subtracted from those of the row pass where
 // that one's length is not 1024) and its transform, A N^2 at k_z = 0, added: it needs no tail
 // beyond the band, and FP32 rows hold no multiple of it (N = 700, central line of I(q): rms error
@@ -1767,28 +1760,28 @@ __global__ __launch_bounds__(BLK) void k_colpass_bsw(gx_frames d, int64_t f0) {
   double2 A = make_double2(0.0, 0.0);
   if (k0 && (d.fill_bkg || d.smooth))
     A = make_double2(d.avg_re * d.max_voxels * (double)N, d.avg_im * d.max_voxels * (double)N);
-  const C a0 = C{(T)A.x, (T)A.y};
+  const C a0 = k0_apart ? C{(T)0, (T)0} : C{(T)A.x, (T)A.y};
   // rows of the band, as in k_colpass_bs (>= Z); without a0, rows from Z on are zero unless
   // smoothing without fill spreads over them
-  const bool head = (d.fill_bkg || !d.smooth) && d.Z <= GX_WAVE * CHW_NZ;
-  const int Lc = (int)min((int64_t)N, d.bs_Mc - d.bs_ck + 1);
+  const bool spread = !d.fill_bkg && d.smooth;  // background beyond the rows of the row pass
+  const int Lc = (int)min((int64_t)N, d.bs_Mc - d.bs_ck + 1), rows = min((int)d.Z, Lc);
   C v[CHW_P];
-  auto load = [&](int q) {
-    const int z = lane + GX_WAVE * q;
-    v[q] = C{(T)0, (T)0};
-    if (z < Lc) {
-      const C e = col_input(d, col, z, false, u, sz_row);  // without A N from row Z on
-      v[q] = cmul(k0_apart || z >= d.Z ? e : csub(e, a0), chirp[z]);
-    }
-  };
-  if (head) {
-#pragma unroll
-    for (int q = 0; q < CHW_NZ; ++q) load(q);
-    DftHead<16, CHW_NZ, C>::run(v);
+  if (spread) {
+    chw_first(v, CHW_M, [&](int q) {
+      const int z = lane + GX_WAVE * q;
+      v[q] = C{(T)0, (T)0};
+      if (z < Lc) {
+        const C e = col_input(d, col, z, false, u, sz_row);  // without A N from row Z on
+        v[q] = cmul(z >= rows ? e : csub(e, a0), chirp[z]);
+      }
+    });
   } else {
-#pragma unroll
-    for (int q = 0; q < CHW_P; ++q) load(q);
-    DftHead<16, CHW_P, C>::run(v);
+    // no branch between the loads: all of them are in flight at once
+    chw_first(v, rows, [&](int q) {
+      const int z = lane + GX_WAVE * q, zc = min(z, rows - 1);
+      const C e = csub(col[zc], a0);
+      v[q] = cmul(z < rows ? e : C{(T)0, (T)0}, chirp[zc]);
+    });
   }
   chirpz_wave<C>(v, lds[wave], reinterpret_cast<const C *>(d.bs_kernel_c),
                  reinterpret_cast<const C *>(d.bs_twiddle_c), lane);
@@ -1929,8 +1922,7 @@ int launch_bs(const gx_frames *d, int64_t f0, int64_t nf, hipStream_t st, bool r
   if (row) {
     switch (d->bs_M) {
       case 1024:
-        return d->bs_rk <= GX_WAVE * CHW_G ? launch_rowpass_bsw<C, CHW_G>(d, f0, nf, st)
-                                           : launch_rowpass_bsw<C, CHW_P>(d, f0, nf, st);
+        return chw_band(d->bs_rk, [&](auto G) { return launch_rowpass_bsw<C, G>(d, f0, nf, st); });
       case 2048: return launch_rowpass_bs_t<2048, C>(d, f0, nf, st);
       case 4096: return launch_rowpass_bs_t<4096, C>(d, f0, nf, st);
     }
@@ -1938,8 +1930,7 @@ int launch_bs(const gx_frames *d, int64_t f0, int64_t nf, hipStream_t st, bool r
     dim3 grid((unsigned)d->W, (unsigned)nf);
     switch (d->bs_Mc) {
       case 1024:
-        return d->bs_ck <= GX_WAVE * CHW_G ? launch_colpass_bsw<C, CHW_G>(d, f0, nf, st)
-                                           : launch_colpass_bsw<C, CHW_P>(d, f0, nf, st);
+        return chw_band(d->bs_ck, [&](auto G) { return launch_colpass_bsw<C, G>(d, f0, nf, st); });
       case 2048: k_colpass_bs<2048, C><<<grid, GX_BLK_FFT, 0, st>>>(*d, f0); return check_launch("k_colpass_bs");
       case 4096: k_colpass_bs<4096, C><<<grid, GX_BLK_FFT, 0, st>>>(*d, f0); return check_launch("k_colpass_bs");
     }
