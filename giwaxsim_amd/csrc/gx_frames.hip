@@ -1008,7 +1008,8 @@ __global__ __launch_bounds__(BLK) void k_rowpass_blk(gx_frames d, int64_t f0, in
 // (spills), while one row per wave is straight-line code (measured on the 1.3M-atom
 // slab: 0.61 ms per 119-frame launch with one row per wave, 1.08 ms with two).  There the waves
 // of a block take the same row of neighbouring frames, so its atoms (78 KB) reach the CU's L1
-// once for the four: 0.61 -> 0.56 ms.  With 8 waves per CU (18 KB of LDS each) the rest is
+// once for the four: 0.61 -> 0.56 ms (frames beyond the last four: 5 frames of a 1.3M-atom slab
+// 0.658 -> 0.640 ms a call against a block with idle waves).  With 8 waves per CU (18 KB of LDS each) the rest is
 // waiting: vector instructions issue 44% of the time.
 template <int N> struct RowRm {
   static constexpr int RPWV = (N <= 1024) ? 8 : 1;
@@ -1030,28 +1031,31 @@ void k_rowpass_rm(gx_frames d, int64_t f0, int64_t nf) {
   int32_t *acc_re = reinterpret_cast<int32_t *>(wbuf);
   int32_t *acc_im = acc_re + N;
 
-  // tile order: frame major, or XCD-aware with the frames of a row block together (bit 2)
-  // (frame, row block); one row per wave: (frames of the block's waves, row)
+  // tile order: frame major, or XCD-aware with the frames of a row block together (bit 2).  With one
+  // row per wave a block takes a row of FW frames; blocks for the frames beyond the last full FW
+  // follow, FW rows of one frame each.
   constexpr int FW = RPWV == 1 ? BLK / GX_WAVE : 1;
-  const int64_t nfg = (nf + FW - 1) / FW, nzb = gridDim.x / nfg;
-  int fb, zb;
-  if (d.row_variant & 4) {
-    const int64_t tile = xcd_tile(blockIdx.x, gridDim.x);
-    fb = (int)(tile % nfg);
-    zb = (int)(tile / nfg);
+  const int64_t nfg = nf / FW, nzb = (d.Z + RB - 1) / RB, n_main = FW > 1 ? d.Z * nfg : gridDim.x;
+  const int64_t tile = (d.row_variant & 4) ? xcd_tile(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x;
+  int fb, zw;  // the wave's frame and first row
+  if (FW > 1 && tile < n_main) {
+    const bool together = d.row_variant & 4;
+    fb = (int)(together ? tile % nfg : tile / d.Z) * FW + wave;
+    zw = (int)(together ? tile / nfg : tile % d.Z);
   } else {
-    fb = (int)(blockIdx.x / nzb);
-    zb = (int)(blockIdx.x % nzb);
+    const int64_t t = FW > 1 ? tile - n_main : tile, n = FW > 1 ? nf - nfg * FW : nf;
+    const bool together = d.row_variant & 4;
+    fb = (int)(nf - n + (together ? t % n : t / nzb));
+    zw = (int)(together ? t / n : t % nzb) * RB + wave * RPWV;
   }
-  if (FW > 1) fb = fb * FW + wave;
-  if (fb >= nf) return;  // wave-uniform, as every return: the kernel has no block barrier
+  // (every return is wave-uniform and the kernel has no block barrier)
   const int64_t f = f0 + fb;
   const double *fp = d.fparams + f * GX_FP_STRIDE;
   const int jlo = (int)fp[GX_FP_JLO], jhi = (int)fp[GX_FP_JHI];
   const int wf = jhi - jlo + 1;
   if (wf <= 0) return;
   if (wf > d.W) {       // planner guarantees wf <= W; never write past a row
-    if (lane == 0 && zb == 0 && (FW > 1 || wave == 0)) atomicAdd(&d.status[1], 1);
+    if (lane == 0 && zw == 0) atomicAdd(&d.status[1], 1);
     return;
   }
   const double s = fp[GX_FP_SIN], c = fp[GX_FP_COS];
@@ -1072,7 +1076,6 @@ void k_rowpass_rm(gx_frames d, int64_t f0, int64_t nf) {
     for (int q = 0; q < R0; ++q)
       my[t * R0 + q] = d.smooth ? (T)d.col_sy[(int64_t)fb * N + lane + GX_WAVE * t + q * (N / R0)] : (T)1;
 
-  const int zw = FW > 1 ? zb : zb * RB + wave * RPWV;
   for (int rr = 0; rr < RPWV; ++rr) {
     const int z = zw + rr;
     if (z >= d.Z) break;
@@ -2035,8 +2038,8 @@ int launch_rowpass_rm_x(const gx_frames *d, int64_t f0, int64_t nf, hipStream_t 
                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     attr_set = true;
   }
-  const unsigned nblk = RPWV == 1 ? (unsigned)(d->Z * ((nf + BLK / GX_WAVE - 1) / (BLK / GX_WAVE)))
-                                  : (unsigned)(((d->Z + RB - 1) / RB) * nf);
+  constexpr int FW = RPWV == 1 ? BLK / GX_WAVE : 1;  // as the kernel
+  const unsigned nblk = (unsigned)((FW > 1 ? d->Z * (nf / FW) : 0) + ((d->Z + RB - 1) / RB) * (FW > 1 ? nf % FW : nf));
   k_rowpass_rm<N, C, RPWV, WPE, PL><<<nblk, BLK, lds, st>>>(*d, f0, nf);
   return check_launch("k_rowpass_rm");
 }
