@@ -192,13 +192,16 @@ def load(path: str | None = None):
     lib.gx_abi_version.argtypes = []
     lib.gx_supported_grid.restype = c_int
     lib.gx_supported_grid.argtypes = [c_int64]
-    for name, args in SIGNATURES.items():
-        fn = getattr(lib, name)
-        fn.restype = c_int
-        fn.argtypes = args
     if lib.gx_abi_version() != GX_ABI_VERSION:
         raise GxError(f"{path} has ABI version {lib.gx_abi_version()}, the binding expects "
                       f"{GX_ABI_VERSION}: rebuild it")
+    for name, args in SIGNATURES.items():
+        try:
+            fn = getattr(lib, name)
+        except AttributeError:
+            raise GxError(f"{path} has no {name}: it is older than the binding, rebuild it") from None
+        fn.restype = c_int
+        fn.argtypes = args
     _lib = lib
     return lib
 
