@@ -7,6 +7,8 @@ import numpy as np
 import pytest
 import torch
 
+import test_gpu_chirpz_wave_adjoint as autograd
+
 from giwaxsim_amd import adjoint, engine
 
 pytestmark = pytest.mark.gpu
@@ -157,3 +159,10 @@ def test_wide_band_fp64():
     engine._WORKSPACES.clear()
     m = got[0] > 1e-6 * got[0].max()
     assert float(((got[1] - got[0]).abs()[m] / got[0][m]).max()) <= 1e-5
+
+
+@pytest.mark.parametrize("fill,smooth", [(False, 0), (True, 3)])
+def test_differentiable_fp64_near_2048(fill, smooth):
+    """FP64 gradients of a small crystal on a large edge, against autograd: the wave-level passes hold
+    rows of 1024 nodes, where the block-wide row gradient would need 4 N."""
+    autograd.test_against_autograd((30.0, 20.0, 16.0), 1990, 0.2, 0.8, fill, smooth, 'CN', 'fp64')
