@@ -287,7 +287,8 @@ int gx_detector_accumulate(const gx_detector *d, gx_stream_t stream);
 /* gx_detector_accumulate, bit for bit and faster, with a 64-byte aligned work buffer for
  * per-orientation linear index maps, which replace the rotations of every sample.
  * gx_detector_work_size gives its size in doubles from the descriptor (host only; 0 where
- * the maps do not apply and the plain kernels run). */
+ * the maps do not apply and the plain kernels run: work may then be NULL).  Both refuse what
+ * gx_detector_accumulate refuses.  Added within version 12, whose structures are unchanged. */
 int gx_detector_work_size(const gx_detector *d, int64_t *n_doubles);
 int gx_detector_accumulate_ws(const gx_detector *d, double *work, gx_stream_t stream);
 /* flags & GX_FIN_MIRROR: mirror_vertical_horizontal (tools/detector.py:246-275);
@@ -567,7 +568,9 @@ int gx_detector_adjoint_mapped(const gx_detector *d, const double *g_out, int64_
  * descriptor field that points to it (0: not needed for this geometry, the field may
  * be NULL).  Per-frame buffers hold `batch` frames (a caller that keeps the statistics
  * of all frames, as the package's engine does, sizes those with batch = n_frames and
- * offsets the descriptor pointers per batch).
+ * offsets the descriptor pointers per batch).  Not among them, as no descriptor field
+ * points to it: the work buffer of gx_detector_accumulate_ws, which gx_detector_work_size
+ * sizes (at most 64 (n_orient + 9) bytes; gx_detector_accumulate takes none).
  * ---------------------------------------------------------------------------------- */
 typedef struct gx_workspace_query {
   int64_t N;               /* real-space grid edge (16..2048) */
